@@ -3,8 +3,8 @@
 // One chunk of n_q queries per (sequence, q-head) attends the sequence's
 // context -- packed 64-token blocks, then an fp16/bf16 tail -- and the chunk's
 // own dense K/V, causally (chunk query i sees chunk tokens 0..i).  The
-// products run in the chunk's dtype: v_mfma_f32_16x16x32_f16 for fp16 data,
-// v_mfma_f32_16x16x32_bf16 for bf16 data (no value is squeezed into the
+// products run in the chunk's dtype: v_mfma_f32_32x32x16_f16 for fp16 data,
+// v_mfma_f32_32x32x16_bf16 for bf16 data (no value is squeezed into the
 // fp16 range); a tail of the other dtype is converted as it is staged.  The
 // reference path materialises the whole K/V (restore of every packed block
 // plus the tail, loop_kv_pk01_cache.py:87-106) and runs dense attention on it;
@@ -12,23 +12,33 @@
 // HBM in dense form.
 //
 // Workgroup = 8 waves = 256 consecutive chunk queries of one (b, q-head);
-// each wave owns 32 queries (two 16-query MFMA column tiles).  Per 64-token
-// block:
+// each wave owns 32 queries (one MFMA column tile).  Per 64-token block:
 //   1. the raw block (K/V codes, K/V min and scale, K/V decode factors; for
 //      a tail or chunk block its dense K/V rows) is staged into LDS by DMA
 //      two blocks ahead;
 //   2. the 512 threads dequantise it once for the workgroup (threads 0-255
 //      K', 256-511 V'^T) into K' [64 tok][128 ch] and V'^T [128 ch][64 tok]
 //      (the reconstructed values f_t * (m + s*z), rounded to the compute
-//      dtype), double-buffered so that the fill of the next block overlaps
-//      the products of this one;
+//      dtype), double-buffered;
 //   3. each wave computes S^T = K' Q^T and O^T += V'^T P^T on MFMA -- the
 //      transposed products keep P in registers: the C layout of S^T is
-//      already the B layout of P^T for a token order in which lane group g
-//      of a 32-token step holds tokens 4g..4g+3 of both 16-token tiles.
+//      already the B layout of P^T for the token order vpos.
 // Softmax runs in the log2 domain: fp16 queries are pre-scaled by
 // scale*log2(e); bf16 queries enter the product exactly and the scores are
 // scaled after it.
+//
+// What bounds it: per wave and block 32 MFMA (1024 cycles), ~130 VALU of fill
+// and ~85 VALU + 32 exp of softmax, on SIMDs that hold two waves each.  While
+// one wave's MFMA runs, the other issues VALU at 58 % of its rate and exp at
+// its full rate (measured), so a SIMD's block takes at least ~3600 cycles
+// with everything overlapped and ~5200 one after the other.  The two waves of
+// a SIMD therefore run half a block out of step (see the block loop).  A late
+// 512-query chunk of a batch (32 sequences, 16 heads, 7680 tokens of context)
+// took 1271 us with 16x16x32 tiles and both waves in step, 1185 us so (at 1.8
+// GHz under the full load); one sequence of 32K tokens, 32 query heads, which
+// loads a quarter of the CUs at 2.3 GHz, 1206 -> 873 us.
+#include <type_traits>
+
 #include "nsn_common.hpp"
 
 namespace nsn {
@@ -38,31 +48,56 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWaves = 8;                // waves per workgroup
 constexpr int kQTile = 32 * kWaves;      // chunk queries per workgroup
-// LDS banking on gfx950 (measured): a ds_read_b128 serves lanes 0-31 and
-// 32-63 in separate passes and is conflict-free when the 32 lanes of a pass
-// hit 32 different 16-byte slots modulo 512 bytes; a ds_write_b32 serves 32
-// lanes per pass over 4-byte slots modulo 128 bytes.
-constexpr int kKP = 144;      // K' row pitch (halves): 288 B rows, so that the S^T operand reads
-                              // (16 rows x 2 lane groups per pass) take 32 different slots
+// LDS banking on gfx950 (measured on the exact patterns): a ds_read_b128 takes
+// 16 lanes a cycle over 16 slots of 16 bytes; lanes 0-3, 12-15, 20-27 share a
+// cycle, the other 16 of lanes 0-31 the next, lanes 32-63 likewise.
+constexpr int kKP = 136;      // K' row pitch (halves): 272 B rows (17 slots), so that the S^T operand
+                              // reads (32 rows, one chunk per pass) take 32 different slots
 constexpr int kVP = 64;       // V'^T row pitch (halves): 128 B rows, slots kept apart by vchunk
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.f;  // running-maximum slack (log2 units): weights < 2^8
 
-// D = A B + C on the compute dtype CT (NSN_DTYPE_F16 or NSN_DTYPE_BF16).
+// D = A B + C on the compute dtype CT (NSN_DTYPE_F16 or NSN_DTYPE_BF16), 32 x
+// 32 x 16.  Lane l (h = l / 32) holds row (column) l % 32 of A (B) at k = 8h ..
+// 8h + 7, and rows 8 (i / 4) + 4h + i % 4 of column l % 32 of C in register i.
 template <int CT>
-__device__ __forceinline__ f32x4 mfma(const u32x4 &a, const u32x4 &b, const f32x4 &c) {
+__device__ __forceinline__ f32x16 mfma(const u32x4 &a, const u32x4 &b, const f32x16 &c) {
     if constexpr (CT == NSN_DTYPE_BF16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                        0, 0);
     else
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
                                                       0);
+}
+// Instruction order of a product loop: N LDS operand reads, each feeding M
+// MFMA, with kAhead reads in flight before the first one (measured: 3 874 us,
+// 4 881 us, 6 887 us, 8 932 us on the single 32K-token sequence; left to the
+// compiler every MFMA waits for its own read).
+constexpr int kAhead = 3;
+template <int N, int M>
+__device__ __forceinline__ void mfma_order() {
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);   // (0x100: LDS reads, 8: MFMA)
+#pragma unroll
+    for (int i = 0; i < N - kAhead; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, M, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x8, M * kAhead, 0);
+}
+// acc + the sum of a packed pair of the compute dtype.
+template <int CT>
+__device__ __forceinline__ float add_pair(uint32_t x, float acc) {
+    if constexpr (CT == NSN_DTYPE_BF16)
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x), __builtin_bit_cast(bf16x2, 0x3F803F80u), acc,
+                                               false);
+    else
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2v, x), __builtin_bit_cast(half2v, 0x3C003C00u), acc, false);
 }
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
     return __builtin_amdgcn_perm(hi, lo, sel);
@@ -78,30 +113,22 @@ __device__ __forceinline__ uint32_t pk(float a, float b) {
         return __builtin_bit_cast(uint32_t, h);
     }
 }
-// Maxima of scores as single v_max3_f32 / v_max_f32 instructions.  fmaxf
-// compiles to the same instructions plus a self-max per operand that the
-// compiler cannot prove canonical (MFMA results, lane swaps): the quieting of
-// signalling NaNs, which a score never is (a NaN score is a quiet NaN out of
-// the MFMA, ignored by the maximum as fmaxf ignores it, and it still reaches
-// the output through its weight).  Half the maximum's instructions were those.
-__device__ __forceinline__ float max3f(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float max2f(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-// Maximum over the four 16-lane rows of the wave (lanes l, l^16, l^32, l^48),
-// on every lane, without LDS: v_permlane16_swap gives rows (0,0,2,2) and
-// (1,1,3,3), v_permlane32_swap the halves (lo,lo) and (hi,hi).
-__device__ __forceinline__ float rows4_max(float x) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = max2f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+// Maxima of scores.  The NaN-propagating maximum is one v_maximum3_f32 with
+// no operand quieted first (fmaxf on MFMA results costs a self-maximum per
+// operand); a NaN score makes its query's output NaN either way.  Not inline
+// asm: the compiler must see that these read MFMA results, which take wait
+// states that the hardware does not insert.
+__device__ __forceinline__ float max2f(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+__device__ __forceinline__ float max3f(float a, float b, float c) { return max2f(max2f(a, b), c); }
+// The two halves of the wave (lanes l and l ^ 32) combined, on every lane,
+// without LDS: v_permlane32_swap gives (lo, lo) and (hi, hi).
+__device__ __forceinline__ float halves_max(float x) {
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return max2f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float halves_sum(float x) {
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 // fp32 pair -> bf16 hi (round to nearest even) + bf16 lo = rn(x - hi): the
 // pair to ~2^-17 relative.
@@ -126,14 +153,13 @@ template <> struct Order<5> {
     static constexpr int kE[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 };
 
-// The 8 codes of one token's 8-channel group, from the staged code bytes:
-// 4 dwords, element p (dword p/2, half p%2) = code of channel chE[p] at bit kE[p].
+// The 8 codes of one token's 8-channel group: bytes BITS*cg .. of its row, in
+// the row's dwords w0 = (BITS*cg)/4 and w1 (the next), from bit sh = 8 *
+// ((BITS*cg) % 4) of w0 -> 4 dwords, element p (dword p/2, half p%2) = code of
+// channel chE[p] at bit kE[p].
 template <int BITS>
-__device__ __forceinline__ void codes8(const uint8_t *row, int cg, uint32_t (&B)[4]) {
-    const int byte = BITS * cg;   // the group's first byte within the token row
-    const uint32_t *w = reinterpret_cast<const uint32_t *>(row + (byte & ~3));
-    const uint32_t sh = 8u * static_cast<uint32_t>(byte & 3);
-    const uint32_t x = __builtin_amdgcn_alignbit(w[1], w[0], sh);
+__device__ __forceinline__ void codes8(uint32_t w0, uint32_t w1, uint32_t sh, uint32_t (&B)[4]) {
+    const uint32_t x = __builtin_amdgcn_alignbit(w1, w0, sh);
     if constexpr (BITS == 3) {
         const uint32_t P = perm(x, x, 0x02010100u), Q = perm(x, x, 0x0C020C02u);
         B[0] = P & 0x000E0007u;
@@ -141,7 +167,7 @@ __device__ __forceinline__ void codes8(const uint8_t *row, int cg, uint32_t (&B)
         B[2] = P & 0x038001C0u;
         B[3] = Q & 0x00E0001Cu;
     } else {
-        const uint32_t y = __builtin_amdgcn_alignbit(w[2], w[1], sh);   // code bits 32..63
+        const uint32_t y = w1 >> sh;   // code bits 32..39
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             uint32_t z[2];
@@ -192,36 +218,43 @@ __device__ __forceinline__ void dma16(const void *src, void *dst) {
 #pragma clang diagnostic pop
 
 // Staged block layout (bytes): [K codes NB | V codes NB | K min 256 | K scale 256 |
-// V min 256 | V scale 256 | K factor 256 | V factor 256].
+// V min 256 | V scale 256 | K factor 256 | V factor 256 | (512 not read)].  K code rows are in
+// token order.  The 16-byte chunk x of V code row t sits at chunk 64x + 16 (t % 4) +
+// t / 4 of its part: the V'^T fill's lanes read rows 4 apart, which in row
+// order fall on two banks.
 template <int BITS> struct Stage {
     static constexpr int NB = packed_block_bytes(BITS);
     static constexpr int META = 2 * NB;
-    static constexpr int BYTES = 2 * NB + 1536;
+    static constexpr int BYTES = 2 * NB + 2048;
     static constexpr int NI = 2 * NB / 1024 + 2;   // 1 KiB DMA instructions per block
+    static constexpr int PER_WAVE = (NI + kWaves - 1) / kWaves;
 };
 
-// DMA of packed block ib of (b, kvh) into one stage; instruction i of the
-// block is issued by wave i % kWaves.
+// One wave's share of the DMA of a packed block: instruction i = wave + 8n of
+// the block.  A lane's source moves by a fixed step per block, so a block's
+// request is one 64-bit multiply-add per instruction.
+struct PackedDma {
+    const uint8_t *src;   // the lane's 16 bytes of block 0 of the stream
+    uint32_t step;        // bytes between two blocks
+    uint32_t dst;         // offset in the stage
+};
 template <int BITS>
-__device__ __forceinline__ void stage_block(const PrefillParams &p, int64_t rk, int64_t rv, int wave, int l,
-                                            uint8_t *st) {
+__device__ __forceinline__ PackedDma packed_dma(const PrefillParams &p, int64_t rk, int64_t rv, int i, int l) {
     using S = Stage<BITS>;
+    constexpr int NK = S::NB / 1024;
     const int q = l & 15;
-    for (int i = wave; i < S::NI; i += kWaves) {
-        if (i < S::NB / 1024) {
-            dma16(p.k.codes + rk * S::NB + 1024 * i + 16 * l, st + 1024 * i);
-        } else if (i < 2 * S::NB / 1024) {
-            const int c = i - S::NB / 1024;
-            dma16(p.v.codes + rv * S::NB + 1024 * c + 16 * l, st + S::NB + 1024 * c);
-        } else if (i == 2 * S::NB / 1024) {
-            const uint16_t *src = (l < 16) ? p.k.mins + rk * kDim : (l < 32) ? p.k.scales + rk * kDim
-                                : (l < 48) ? p.v.mins + rv * kDim : p.v.scales + rv * kDim;
-            dma16(src + 8 * q, st + S::META);
-        } else if (l < 32) {
-            const float *src = (l < 16) ? p.k.factors + rk * kBlockTok : p.v.factors + rv * kBlockTok;
-            dma16(src + 4 * q, st + S::META + 1024);
-        }
+    if (i < NK) return {p.k.codes + rk * S::NB + 1024 * i + 16 * l, S::NB, 1024u * i};
+    if (i < 2 * NK) {
+        const int x = i - NK, t = 4 * q + (l >> 4);
+        return {p.v.codes + rv * S::NB + (S::NB / kBlockTok) * t + 16 * x, S::NB, 1024u * i};
     }
+    if (i == 2 * NK) {
+        const uint16_t *m = (l < 16) ? p.k.mins + rk * kDim : (l < 32) ? p.k.scales + rk * kDim
+                          : (l < 48) ? p.v.mins + rv * kDim : p.v.scales + rv * kDim;
+        return {reinterpret_cast<const uint8_t *>(m + 8 * q), 2 * kDim, S::META};
+    }
+    const float *f = (l & 16) ? p.v.factors + rv * kBlockTok : p.k.factors + rk * kBlockTok;   // (lanes 32-63: again)
+    return {reinterpret_cast<const uint8_t *>(f + 4 * q), 4 * kBlockTok, S::META + 1024};
 }
 
 // A dense block (tail or chunk tokens, 2-byte elements) is staged by DMA
@@ -248,30 +281,31 @@ __device__ __forceinline__ void stage_dense(const uint16_t *xk, const uint16_t *
 }
 
 // V'^T keeps each channel's 64 tokens in the k order of the PV product:
-// token t = 32a + 16h + 4g + i sits at position 32a + 8g + 4h + i, so the 8
-// tokens that lane group g of 32-token step a contracts (4g..4g+3 of both
-// 16-token tiles) are one 16-byte read.  Groups of 4 tokens stay together.
-__device__ __forceinline__ int vpos(int t) {
-    return (t & 32) | ((t & 12) << 1) | ((t & 16) >> 2) | (t & 3);
-}
+// token t = 16c + 8a + 4h + i sits at position 16c + 8h + 4a + i, so the 8
+// tokens that half h of the wave contracts in 16-token step c (the rows of
+// S^T that its registers hold) are one 16-byte read.  Groups of 4 stay together.
+__device__ __forceinline__ int vpos(int t) { return (t & 51) | ((t & 4) << 1) | ((t & 8) >> 1); }
 
-// V'^T row `r` keeps its 16-byte chunk c at position c ^ x(r), x(r) = 4 * bit 2
-// of r + 2 * bit 3 of r.  Rows are 128 B, so rows r, r+4, r+8, r+12 start on
-// the same banks:
-//  - a PV operand read pass (rows 16*ct + 0..15, chunks c and c+1) gives
-//    those four rows four different XORs in {0, 2, 4, 6}: 32 different slots;
-//  - a fill write pass (32 lanes: 16 token groups of rows r and r+8) writes,
-//    in each 16-byte chunk, the two words whose parity is bit 1 of the
-//    chunk's index (fill_packed's pair order); x(r+8) = x(r) ^ 2 flips that
-//    bit, so row r+8 writes the other two words of every chunk position and
-//    the pass takes 32 different banks.
-__device__ __forceinline__ int vchunk(int r, int c) { return c ^ ((r & 4) | ((r >> 2) & 2)); }
+// V'^T row `r` keeps its 16-byte chunk c at position c ^ ((r >> 1) & 7).  Rows
+// are 128 B, half a pass of the banks: of the rows that one pass of a PV
+// operand read takes (0-3, 12-15, 20-27 or the other 16 of 32), the eight of
+// each parity get eight different slots (the measured cycles of the exact
+// pattern equal a linear read's; r >> 2 is 2-way).  A fill write pass (16
+// token groups of one row) writes a whole row.
+__device__ __forceinline__ int vchunk(int r, int c) { return c ^ ((r >> 1) & 7); }
 __device__ __forceinline__ int vcol_at(int r, int t) { return 8 * vchunk(r, vpos(t) >> 3) + (vpos(t) & 7); }
 
 // The block buffer compute reads: K' [64 tok][kKP], V'^T [128 ch][kVP].
+// A fill thread's place in it: K' rows 4*rg .. +3 from kt (channels 8*cg ..);
+// V'^T rows 8*cg + c (c = 0 .. 7), tokens 4*rg .. +3, at vt + vx[c / 2] + c * kVP
+// (the chunk XOR of row 8*cg + c is that of row 8*cg with c / 2 on top).
 struct KV {
     uint16_t *kt, *vt;
+    uint32_t vx[4];
 };
+__device__ __forceinline__ void store_vcol(const KV &kv, int c, const uint32_t (&w)[2]) {
+    *reinterpret_cast<u32x2 *>(kv.vt + kv.vx[c >> 1] + c * kVP) = u32x2{w[0], w[1]};
+}
 
 // Fill one side of a KV buffer from a staged dense block of dtype DT
 // (`valid` rows; rows past it are zero), rounded to CT.  Thread: tokens
@@ -320,8 +354,7 @@ __device__ __forceinline__ void fill_dense(const uint8_t *st, int valid, int rg,
     if constexpr (side == 1) {
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-            *reinterpret_cast<u32x2 *>(kv.vt + (8 * cg + e) * kVP + vcol_at(8 * cg + e, 4 * rg)) =
-                u32x2{vcol[e][0], vcol[e][1]};
+            store_vcol(kv, e, vcol[e]);
     }
 }
 
@@ -345,46 +378,42 @@ __device__ __forceinline__ void fill_packed(const uint8_t *st, int rg, int cg, c
     for (int p = 0; p < 8; ++p) {
         const int c = O::chE[p];
         mE[p] = h16(M[c >> 1], c & 1);
-        sE[p] = h16(SC[c >> 1], c & 1) * static_cast<float>(1u << (24 - O::kE[p]));
+        sE[p] = __builtin_fmaf(h16(SC[c >> 1], c & 1), static_cast<float>(1u << (24 - O::kE[p])), 0.f);   // (one fma_mix)
     }
-    const uint8_t *codes = st + S::NB * side;
-    // V side (lanes = token groups): rows 4*rg are 48 B = 16 banks apart, so
-    // the lanes of a pass alternate the order of their two token pairs
-    // (4-way instead of 8-way bank sharing on the code reads).  Register slot
-    // s holds pair s ^ pfirst; only the addresses change.
-    const int pfirst = (side == 1) ? ((rg >> 1) & 1) : 0;
+    const int byte = BITS * cg, d0 = byte >> 2;
+    const uint32_t sh = 8u * static_cast<uint32_t>(byte & 3);
+    // token 4*rg + i's dwords d0 and d0 + 1 (past the last group's row: the
+    // next row or part, whose bits are shifted out)
+    auto vdw = [&](int d) { return S::NB + 1024 * (d >> 2) + 16 * rg + 4 * (d & 3); };
+    const uint8_t *c0 = st + (side ? vdw(d0) : ROWB * 4 * rg + 4 * d0);
+    const uint8_t *c1 = st + (side ? vdw(d0 + 1) : ROWB * 4 * rg + 4 * d0 + 4);
+    constexpr int PITCH = side ? 256 : ROWB;
     uint32_t vcol[8][2];
     float vprev[8];
 #pragma unroll
-    for (int slot = 0; slot < 2; ++slot) {
+    for (int i = 0; i < 4; ++i) {
+        const int t = 4 * rg + i;
+        uint32_t b[4];
+        codes8<BITS>(*reinterpret_cast<const uint32_t *>(c0 + PITCH * i), *reinterpret_cast<const uint32_t *>(c1 + PITCH * i),
+                     sh, b);
+        float d[8];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int t = 4 * rg + 2 * (slot ^ pfirst) + h;
-            const float ft = pfirst ? fac[2 * (slot ^ 1) + h] : fac[2 * slot + h];
-            uint32_t b[4];
-            codes8<BITS>(codes + t * ROWB, cg, b);
-            float d[8];
+        for (int p = 0; p < 8; ++p) d[p] = __builtin_fmaf(h16(b[p >> 1], p & 1), sE[p], mE[p]) * fac[i];
+        if constexpr (side == 0) {
+            *reinterpret_cast<uint4 *>(kv.kt + t * kKP + 8 * cg) =
+                uint4{pk<CT>(d[0], d[1]), pk<CT>(d[2], d[3]), pk<CT>(d[4], d[5]), pk<CT>(d[6], d[7])};
+        } else {
 #pragma unroll
-            for (int p = 0; p < 8; ++p) d[p] = __builtin_fmaf(h16(b[p >> 1], p & 1), sE[p], mE[p]) * ft;
-            if constexpr (side == 0) {
-                *reinterpret_cast<uint4 *>(kv.kt + t * kKP + 8 * cg) =
-                    uint4{pk<CT>(d[0], d[1]), pk<CT>(d[2], d[3]), pk<CT>(d[4], d[5]), pk<CT>(d[6], d[7])};
-            } else {
-#pragma unroll
-                for (int p = 0; p < 8; ++p) {
-                    if (h) vcol[p][slot] = pk<CT>(vprev[p], d[p]);
-                    else vprev[p] = d[p];
-                }
+            for (int p = 0; p < 8; ++p) {
+                if (i & 1) vcol[p][i >> 1] = pk<CT>(vprev[p], d[p]);
+                else vprev[p] = d[p];
             }
         }
     }
     if constexpr (side == 1) {
 #pragma unroll
-        for (int p = 0; p < 8; ++p) {
-            uint16_t *dst = kv.vt + (8 * cg + O::chE[p]) * kVP + vcol_at(8 * cg + O::chE[p], 4 * rg);
-            *reinterpret_cast<uint32_t *>(dst + 2 * pfirst) = vcol[p][0];
-            *reinterpret_cast<uint32_t *>(dst + 2 * (pfirst ^ 1)) = vcol[p][1];
-        }
+        for (int p = 0; p < 8; ++p)
+            store_vcol(kv, O::chE[p], vcol[p]);
     }
 }
 
@@ -407,7 +436,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
 
     const int tid = threadIdx.x, l = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (uniform: the DMA targets are scalar)
-    const int row = l & 15, g = l >> 4;
+    const int col = l & 31, h = l >> 5;
     // fill role: threads 0..255 fill K' (lanes over channel groups: each pass
     // writes whole K' rows), 256..511 V'^T (lanes over token groups: each pass
     // writes one contiguous V'^T row)
@@ -424,47 +453,44 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     const int64_t qw = q0 + 32 * wave;                     // this wave's first query
     const int64_t seqrow = static_cast<int64_t>(b) * p.heads_kv + kvh;
 
-    // ---- Q fragments (B operand of S^T = K' Q^T): query qw + 16*qt + row,
-    // channels 32*ks + 8*g + chE[e] (fp16: times scale*log2(e)); loaded
-    // before the context lengths are needed, so the two round trips overlap
-    u32x4 qf[2][4];
+    // ---- Q fragments (B operand of S^T = K' Q^T): query qw + l % 32, channels
+    // 16*ks + 8*h + chE[e] (fp16: times scale*log2(e)); loaded before the
+    // context lengths are needed, so the two round trips overlap
+    u32x4 qf[8];
+    const int64_t qi = qw + col;   // this lane's query
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-        const int64_t qi = qw + 16 * qt + row;
+    for (int ks = 0; ks < 8; ++ks) {
+        float x[8];
+        if (qi < p.n_q) {
+            const uint4 a = *reinterpret_cast<const uint4 *>(
+                p.q + ((static_cast<int64_t>(b) * p.heads_q + hq) * p.n_q + qi) * kDim + 16 * ks + 8 * h);
+            const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            float x[8];
-            if (qi < p.n_q) {
-                const uint4 a = *reinterpret_cast<const uint4 *>(
-                    p.q + ((static_cast<int64_t>(b) * p.heads_q + hq) * p.n_q + qi) * kDim + 32 * ks + 8 * g);
-                const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    x[e] = Elem<DT>::load(static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1))));
-                    if (QPRE) x[e] *= p.qscale;
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = 0.f;
+            for (int e = 0; e < 8; ++e) {
+                x[e] = Elem<DT>::load(static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1))));
+                if (QPRE) x[e] *= p.qscale;
             }
-            qf[qt][ks] = u32x4{pk<DT>(x[O::chE[0]], x[O::chE[1]]), pk<DT>(x[O::chE[2]], x[O::chE[3]]),
-                               pk<DT>(x[O::chE[4]], x[O::chE[5]]), pk<DT>(x[O::chE[6]], x[O::chE[7]])};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = 0.f;
         }
+        qf[ks] = u32x4{pk<DT>(x[O::chE[0]], x[O::chE[1]]), pk<DT>(x[O::chE[2]], x[O::chE[3]]),
+                       pk<DT>(x[O::chE[4]], x[O::chE[5]]), pk<DT>(x[O::chE[6]], x[O::chE[7]])};
     }
 
     const int64_t T = p.ctx_len[b];
     const int64_t nbk = p.k.blocks ? p.k.blocks[b] : 0;
     const int64_t nbv = p.v.blocks ? p.v.blocks[b] : 0;
-    const int64_t nb = nbk;                                // (== nbv, checked below)
-    const int64_t ntail = T - nb * kBlockTok;
-    const int64_t qend = (q0 + kQTile < p.n_q) ? q0 + kQTile : p.n_q;   // chunk tokens this workgroup sees
-    const int64_t nt_blk = (ntail + kBlockTok - 1) / kBlockTok;
-    const int64_t nblk = nb + nt_blk + (qend + kBlockTok - 1) / kBlockTok;
-    if (nbk != nbv || nb < 0 || (nb > 0 && (nb > p.k.block_cap || nb > p.v.block_cap)) || ntail < 0 ||
-        ntail > p.k.tail_cap || ntail > p.v.tail_cap) {
+    if (nbk != nbv || nbk < 0 || (nbk > 0 && (nbk > p.k.block_cap || nbk > p.v.block_cap)) || T - nbk * kBlockTok < 0 ||
+        T - nbk * kBlockTok > p.k.tail_cap || T - nbk * kBlockTok > p.v.tail_cap) {
         if (tid == 0) raise_status(p.status, NSN_ST_CAPACITY);   // inconsistent cache (host checks first)
         return;
     }
+    const int nb = static_cast<int>(nbk), ntail = static_cast<int>(T - nbk * kBlockTok);
+    const int nq = static_cast<int>(p.n_q);                      // (< 2^24: the grid's limit)
+    const int qend = (q0 + kQTile < nq) ? static_cast<int>(q0) + kQTile : nq;   // chunk tokens this workgroup sees
+    const int nt_blk = static_cast<int>((static_cast<int64_t>(ntail) + kBlockTok - 1) / kBlockTok);
+    const int nblk = nb + nt_blk + (qend + kBlockTok - 1) / kBlockTok;
     // append: the workgroup of the last query tile (it stages every chunk
     // block) of each kv-head's first q-head writes the chunk's K/V to tail
     // rows ntail .. ntail + n_q - 1 as it fills them; no room: flag, no append
@@ -472,65 +498,72 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     const bool app_ok = app_wg && ntail + p.n_q <= p.k.tail_cap && ntail + p.n_q <= p.v.tail_cap;
     if (app_wg && !app_ok && tid == 0) raise_status(p.status, NSN_ST_CAPACITY);
 
-    f32x4 acc[8][2];   // O^T tiles [channel tile ct][query tile qt]
+    f32x16 acc[4];   // O^T tiles: channels 32*ct + 8*(i/4) + 4*h + i%4 of query qi
 #pragma unroll
-    for (int ct = 0; ct < 8; ++ct)
+    for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) acc[ct][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m_run[2] = {-INFINITY, -INFINITY};
-    // Row sums of the weights on the matrix core: a constant A tile whose row
-    // 0 is all ones, so row 0 of lsum[qt] = sum over tokens of the P operand
-    // (the rounded weights the PV product uses); lanes 0-15 hold it.
-    f32x4 lsum[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    const uint32_t one2 = (row == 0) ? (DT == NSN_DTYPE_BF16 ? 0x3F803F80u : 0x3C003C00u) : 0u;
-    const u32x4 ones_a = u32x4{one2, one2, one2, one2};
+        for (int i = 0; i < 16; ++i) acc[ct][i] = 0.f;
+    float m_run = -INFINITY;
+    float lsum = 0.f;   // sum of the rounded weights of this lane's tokens (half of the query's)
     bool bad = false;
+    const bool live = qw < p.n_q;   // (a wave past the chunk end only helps stage and fill)
 
     // Block j: packed (j < nb), tail (nb <= j < nb + nt_blk), or chunk; its rows
     // in use and (chunk blocks) the chunk position of its first token.
-    auto block_rows = [&](int64_t j, int &valid, int64_t &cpos) {
+    auto block_rows = [&](int j, int &valid, int &cpos) __attribute__((always_inline)) {
         cpos = -1;
         if (j < nb) {
             valid = kBlockTok;
         } else if (j < nb + nt_blk) {
-            const int64_t t0 = (j - nb) * kBlockTok;
-            valid = static_cast<int>((ntail - t0 < kBlockTok) ? ntail - t0 : kBlockTok);
+            const int t0 = (j - nb) * kBlockTok;
+            valid = (ntail - t0 < kBlockTok) ? ntail - t0 : kBlockTok;
         } else {
             cpos = (j - nb - nt_blk) * kBlockTok;
-            valid = static_cast<int>((qend - cpos < kBlockTok) ? qend - cpos : kBlockTok);
+            valid = (qend - cpos < kBlockTok) ? qend - cpos : kBlockTok;
         }
     };
-    // Fill block j into KV buffer j & 1 (its raw stage j & 1 when packed).
-    auto fill = [&](int64_t j) {
-        const KV kv{kt[j & 1], vt[j & 1]};
-        if (j < nb) {
-            if (side) fill_packed<BITS, DT, 1>(stg[j & 1], rg, cg, kv);
-            else fill_packed<BITS, DT, 0>(stg[j & 1], rg, cg, kv);
+    uint32_t vx[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) vx[x] = 8 * cg * kVP + vcol_at(8 * cg + 2 * x, 4 * rg);
+    // Fill side SIDE of block j (K' or V'^T) into buffer j & 1 from its raw stage j & 1.
+    auto fill = [&](auto side_c, auto packed_c, int j) __attribute__((always_inline)) {
+        constexpr int SIDE = decltype(side_c)::value;
+        constexpr bool PACKED = decltype(packed_c)::value;
+        const KV kv{kt[j & 1], vt[j & 1], {vx[0], vx[1], vx[2], vx[3]}};
+        if (PACKED || j < nb) {
+            fill_packed<BITS, DT, SIDE>(stg[j & 1], rg, cg, kv);
+            if (!PACKED) asm volatile("; packed block filled");   // (keeps the two paths' stores apart: merged, they cost address moves)
         } else {
             int valid;
-            int64_t cpos;
+            int cpos;
             block_rows(j, valid, cpos);
             if (cpos < 0) {
-                if (side) fill_dense<BITS, TDT, DT, 1, TDT>(stg[j & 1], valid, rg, cg, kv, nullptr);
-                else fill_dense<BITS, TDT, DT, 0, TDT>(stg[j & 1], valid, rg, cg, kv, nullptr);
+                fill_dense<BITS, TDT, DT, SIDE, TDT>(stg[j & 1], valid, rg, cg, kv, nullptr);
             } else {
                 uint16_t *app = nullptr;
                 if (app_ok)
-                    app = side ? p.va + (seqrow * p.v.tail_cap + ntail + cpos) * kDim
+                    app = SIDE ? p.va + (seqrow * p.v.tail_cap + ntail + cpos) * kDim
                                : p.ka + (seqrow * p.k.tail_cap + ntail + cpos) * kDim;
-                if (side) fill_dense<BITS, DT, DT, 1, TDT>(stg[j & 1], valid, rg, cg, kv, app);
-                else fill_dense<BITS, DT, DT, 0, TDT>(stg[j & 1], valid, rg, cg, kv, app);
+                fill_dense<BITS, DT, DT, SIDE, TDT>(stg[j & 1], valid, rg, cg, kv, app);
             }
         }
     };
+    PackedDma pdma[S::PER_WAVE];
+#pragma unroll
+    for (int n = 0; n < S::PER_WAVE; ++n)
+        pdma[n] = packed_dma<BITS>(p, seqrow * p.k.block_cap, seqrow * p.v.block_cap, wave + kWaves * n, l);
     // Stage the raw data of block j into stage j & 1: packed codes and
     // metadata, or the valid rows of its tail / chunk tokens.
-    auto stage = [&](int64_t j) {
-        if (j < nb) {
-            stage_block<BITS>(p, seqrow * p.k.block_cap + j, seqrow * p.v.block_cap + j, wave, l, stg[j & 1]);
+    auto stage = [&](auto packed_c, int j) __attribute__((always_inline)) {
+        if (decltype(packed_c)::value || j < nb) {
+#pragma unroll
+            for (int n = 0; n < S::PER_WAVE; ++n)
+                if (wave + kWaves * n < S::NI)
+                    dma16(pdma[n].src + static_cast<uint64_t>(static_cast<uint32_t>(j)) * pdma[n].step,
+                          stg[j & 1] + pdma[n].dst);
         } else {
             int valid;
-            int64_t cpos;
+            int cpos;
             block_rows(j, valid, cpos);
             if (cpos < 0) {
                 const int64_t t0 = (j - nb) * kBlockTok;
@@ -543,146 +576,191 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
         }
     };
 
-    // ---- prologue: raw blocks 0 and 1 staged together (one round trip), block 0 filled
-    stage(0);
-    if (nblk > 1) stage(1);
+    // ---- S^T[token][query] = K' Q^T: register i of s[tt] holds token
+    // 32*tt + 8*(i/4) + 4*h + i%4
+    f32x16 s[2];
+    auto scores = [&](int j) __attribute__((always_inline)) {
+        const uint16_t *ktj = kt[j & 1] + col * kKP + 8 * h;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[tt][i] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                const u32x4 a = *reinterpret_cast<const u32x4 *>(ktj + 32 * tt * kKP + 16 * ks);
+                s[tt] = mfma<DT>(a, qf[ks], s[tt]);
+            }
+        mfma_order<16, 1>();
+    };
+    // ---- online softmax of the lane's query.  The running maximum (and the
+    // state's rescale) only moves when some lane's block maximum passes it by
+    // more than kLazy (log2 units): weights then stay below 2^kLazy, which
+    // every weight form holds exactly as well as weights below 1.
+    u32x4 pb[4];              // P''^T B operands of the 16-token steps (LO: the bf16 hi parts)
+    u32x4 pl[LO ? 4 : 1];     // LO: the bf16 lo parts
+    auto softmax = [&](auto packed_c, int j) __attribute__((always_inline)) {
+        int valid = kBlockTok;
+        int cpos = -1;
+        if (!decltype(packed_c)::value) block_rows(j, valid, cpos);
+        if (valid < kBlockTok || cpos >= 0) {   // (uniform) partial or causal block
+            // allowed tokens of this block: tok < valid and (chunk blocks) tok <= query - cpos
+            const int rel = (cpos >= 0) ? static_cast<int>(qi) - cpos : kBlockTok;
+            const int lim = (rel < valid - 1) ? rel : valid - 1;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (32 * tt + 8 * (i >> 2) + 4 * h + (i & 3) > lim) s[tt][i] = -INFINITY;
+        }
+        float mx = max2f(s[0][15], s[1][15]);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            const float a0 = max3f(s[tt][0], s[tt][1], s[tt][2]), a1 = max3f(s[tt][3], s[tt][4], s[tt][5]);
+            const float a2 = max3f(s[tt][6], s[tt][7], s[tt][8]), a3 = max3f(s[tt][9], s[tt][10], s[tt][11]);
+            const float a4 = max3f(s[tt][12], s[tt][13], s[tt][14]);
+            mx = max3f(mx, max3f(a0, a1, a2), max2f(a3, a4));
+        }
+        mx = halves_max(mx);
+        if (!QPRE) mx *= p.qscale;   // (bf16: the scores scale inside the exponent below)
+        if (__builtin_amdgcn_ballot_w64(mx > m_run + kLazy)) {
+            const float mnew = fmaxf(m_run, mx);
+            const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - mnew);
+            lsum *= alpha;
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct) acc[ct] *= alpha;
+            m_run = mnew;
+        }
+        const float msafe = (m_run == -INFINITY) ? 0.f : m_run;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float w[2];
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const float v = s[c >> 1][8 * (c & 1) + 2 * e + x];
+                    w[x] = __builtin_amdgcn_exp2f(QPRE ? v - msafe : __builtin_fmaf(v, p.qscale, -msafe));
+                }
+                if constexpr (LO) split_bf16(w[0], w[1], hi[e], lo[e]);
+                else hi[e] = pk<DT>(w[0], w[1]);
+                // the row sum takes the rounded weights that the PV product uses
+                lsum = add_pair<DT>(hi[e], lsum);
+                if constexpr (LO) lsum = add_pair<DT>(lo[e], lsum);
+            }
+            pb[c] = u32x4{hi[0], hi[1], hi[2], hi[3]};
+            if constexpr (LO) pl[c] = u32x4{lo[0], lo[1], lo[2], lo[3]};
+        }
+    };
+    // ---- O^T[channel][query] += V'^T P''^T over the block's four 16-token steps
+    auto output = [&](int j) __attribute__((always_inline)) {
+        const uint16_t *vtj = vt[j & 1] + col * kVP;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct) {   // (row 32*ct + col: the same XOR for every ct)
+                const u32x4 a = *reinterpret_cast<const u32x4 *>(vtj + 32 * ct * kVP + 8 * vchunk(col, 2 * c + h));
+                acc[ct] = mfma<DT>(a, pb[c], acc[ct]);
+                if constexpr (LO) acc[ct] = mfma<DT>(a, pl[c], acc[ct]);
+            }
+        mfma_order<16, LO ? 2 : 1>();
+    };
+    auto barrier = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    using F_ = std::false_type;
+    using T_ = std::true_type;
+    using K_ = std::integral_constant<int, 0>;
+    using V_ = std::integral_constant<int, 1>;
+
+    // ---- prologue: raw blocks 0 and 1 staged together (one round trip), K' of block 0 filled
+    stage(F_{}, 0);
+    if (nblk > 1) stage(F_{}, 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    fill(0);
+    if (side == 0) fill(K_{}, F_{}, 0);
+    barrier();
 
-    // ---- one barrier per block: compute block j from KV buffer j & 1 while
-    // filling block j + 1 into the other and staging raw block j + 2
-    for (int64_t j = 0; j < nblk; ++j) {
-        // KV buffer j & 1 is filled, raw block j + 1 is in, buffer (j + 1) & 1
-        // and raw stage j & 1 are free
+    // ---- The two waves of a SIMD (w and w + 4) run half a block out of step,
+    // so that one's MFMA work meets the other's VALU work.  Per block j:
+    //   first half    waves 0-3: S^T(j), softmax(j)    waves 4-7: fill V'^T(j), O^T(j-1)
+    //   second half   waves 0-3: fill K'(j+1), O^T(j)  waves 4-7: S^T(j), softmax(j)
+    // K'(j+1) goes into the buffer whose last readers (S^T(j-1)) are a half
+    // block back, V'^T(j) into the one that O^T(j-2) left; raw block j + 2 is
+    // requested when V'^T(j) has been read and waited for before K'(j+2).
+    // Priorities: a fill goes before the other wave's softmax (and its own
+    // products come right behind it), so that the products overlap the rest of
+    // that softmax; without priorities the older waves win every conflict and
+    // the late chunk takes 1224 us instead of 1160.  The packed stretch (blocks
+    // j .. j + 2 packed) has a loop of its own: its body has no branch on the
+    // block kind.
+    auto attend = [&](auto packed_c, int j) __attribute__((always_inline)) {
+        if (!live) return;
+        __builtin_amdgcn_s_setprio(2);
+        scores(j);
+        __builtin_amdgcn_s_setprio(0);
+        softmax(packed_c, j);
+    };
+    auto step_k = [&](auto packed_c, int j) __attribute__((always_inline)) {
+        constexpr bool PACKED = decltype(packed_c)::value;
+        attend(packed_c, j);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // raw block j + 1
+        barrier();
+        if (PACKED || j + 2 < nblk) stage(packed_c, j + 2);
+        __builtin_amdgcn_s_setprio(3);
+        if (PACKED || j + 1 < nblk) fill(K_{}, packed_c, j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(3);
+        if (live) output(j);
+        barrier();
+    };
+    auto step_v = [&](auto packed_c, int j) __attribute__((always_inline)) {
+        constexpr bool PACKED = decltype(packed_c)::value;
+        __builtin_amdgcn_s_setprio(3);
+        fill(V_{}, packed_c, j);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(3);
+        if (live && j > 0) output(j - 1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (j + 2 < nblk) stage(j + 2);
-        if (j + 1 < nblk) fill(j + 1);
-        if (qw >= p.n_q) continue;   // (a wave past the chunk end only helps fill)
-        int valid;
-        int64_t cpos;
-        block_rows(j, valid, cpos);
-        const uint16_t *ktj = kt[j & 1];
-        const uint16_t *vtj = vt[j & 1];
-
-        // ---- S^T[token][query] = K' Q^T
-        f32x4 s[4][2];
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-#pragma unroll
-            for (int qt = 0; qt < 2; ++qt) s[tt][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const u32x4 a = *reinterpret_cast<const u32x4 *>(ktj + (16 * tt + row) * kKP + 32 * ks + 8 * g);
-#pragma unroll
-                for (int qt = 0; qt < 2; ++qt) s[tt][qt] = mfma<DT>(a, qf[qt][ks], s[tt][qt]);
-            }
-        }
-        // ---- online softmax per query (lane's query qw + 16*qt + row).  The
-        // running maximum (and the state's rescale) only moves when some
-        // lane's block maximum exceeds it.
-        const bool masked = valid < kBlockTok || cpos >= 0;   // (uniform) partial or causal block
-        u32x4 pb[2][2];   // P''^T B operands [ks2][qt] (LO: the bf16 hi parts)
-        u32x4 pl[2][2];   // LO: the bf16 lo parts
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-            if (masked) {
-                // allowed tokens of this block: tok < valid and (chunk blocks) tok <= query - cpos
-                const int64_t rel = (cpos >= 0) ? qw + 16 * qt + row - cpos : kBlockTok;
-                const int lim = static_cast<int>((rel < valid - 1) ? rel : valid - 1);
-#pragma unroll
-                for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (16 * tt + 4 * g + i > lim) s[tt][qt][i] = -INFINITY;
-            }
-            const f32x4 *v = &s[0][qt];   // (stride 2: s[tt][qt] = v[2 * tt])
-            const float a0 = max3f(v[0][0], v[0][1], v[0][2]), a1 = max3f(v[0][3], v[2][0], v[2][1]);
-            const float a2 = max3f(v[2][2], v[2][3], v[4][0]), a3 = max3f(v[4][1], v[4][2], v[4][3]);
-            const float a4 = max3f(v[6][0], v[6][1], v[6][2]);
-            float mx = max2f(max3f(a0, a1, a2), max3f(a3, a4, v[6][3]));
-            mx = rows4_max(mx);
-            if (!QPRE) mx *= p.qscale;   // (bf16: the scores scale inside the exponent below)
-            // The running maximum moves only when a score passes it by more
-            // than kLazy (log2 units): weights then stay below 2^kLazy, which
-            // every weight form holds exactly as well as weights below 1.
-            if (__builtin_amdgcn_ballot_w64(mx > m_run[qt] + kLazy)) {
-                const float mnew = fmaxf(m_run[qt], mx);
-                const float alpha = (m_run[qt] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run[qt] - mnew);
-                lsum[qt] *= alpha;
-#pragma unroll
-                for (int ct = 0; ct < 8; ++ct) acc[ct][qt] *= alpha;
-                m_run[qt] = mnew;
-            }
-            const float msafe = (m_run[qt] == -INFINITY) ? 0.f : m_run[qt];
-            float pw[4][4];
-#pragma unroll
-            for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    pw[tt][i] = __builtin_amdgcn_exp2f(QPRE ? s[tt][qt][i] - msafe
-                                                            : __builtin_fmaf(s[tt][qt][i], p.qscale, -msafe));
-#pragma unroll
-            for (int ks2 = 0; ks2 < 2; ++ks2) {
-                if constexpr (LO) {
-                    uint32_t h[4], lo[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        split_bf16(pw[2 * ks2 + (e >> 1)][2 * (e & 1)], pw[2 * ks2 + (e >> 1)][2 * (e & 1) + 1], h[e],
-                                   lo[e]);
-                    pb[ks2][qt] = u32x4{h[0], h[1], h[2], h[3]};
-                    pl[ks2][qt] = u32x4{lo[0], lo[1], lo[2], lo[3]};
-                } else {
-                    pb[ks2][qt] = u32x4{pk<DT>(pw[2 * ks2][0], pw[2 * ks2][1]), pk<DT>(pw[2 * ks2][2], pw[2 * ks2][3]),
-                                        pk<DT>(pw[2 * ks2 + 1][0], pw[2 * ks2 + 1][1]),
-                                        pk<DT>(pw[2 * ks2 + 1][2], pw[2 * ks2 + 1][3])};
-                }
-            }
-        }
-        // ---- O^T[channel][query] += V'^T P''^T (k order: tokens 4g..4g+3 of both 16-token tiles)
-#pragma unroll
-        for (int ct = 0; ct < 8; ++ct) {
-#pragma unroll
-            for (int ks2 = 0; ks2 < 2; ++ks2) {
-                const u32x4 a = *reinterpret_cast<const u32x4 *>(vtj + (16 * ct + row) * kVP +
-                                                                 8 * vchunk(16 * ct + row, 4 * ks2 + g));
-#pragma unroll
-                for (int qt = 0; qt < 2; ++qt) {
-                    acc[ct][qt] = mfma<DT>(a, pb[ks2][qt], acc[ct][qt]);
-                    if constexpr (LO) acc[ct][qt] = mfma<DT>(a, pl[ks2][qt], acc[ct][qt]);
-                }
-            }
-        }
-#pragma unroll
-        for (int ks2 = 0; ks2 < 2; ++ks2)
-#pragma unroll
-            for (int qt = 0; qt < 2; ++qt) {
-                lsum[qt] = mfma<DT>(ones_a, pb[ks2][qt], lsum[qt]);
-                if constexpr (LO) lsum[qt] = mfma<DT>(ones_a, pl[ks2][qt], lsum[qt]);
-            }
+        barrier();
+        if (PACKED || j + 2 < nblk) stage(packed_c, j + 2);
+        attend(packed_c, j);
+        barrier();
+    };
+    int j = 0;
+    if (side == 0) {
+        for (; j + 2 < nb; ++j) step_k(T_{}, j);
+        for (; j < nblk; ++j) step_k(F_{}, j);
+    } else {
+        for (; j + 2 < nb; ++j) step_v(T_{}, j);
+        for (; j < nblk; ++j) step_v(F_{}, j);
+        if (live) output(nblk - 1);
     }
 
-    // ---- output: O[q][c] = O^T / l, channels 16*ct + 4*g + i of query qw + 16*qt + row
-#pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-        const float lt = __shfl(lsum[qt][0], row);   // (query row's sum, from lane row)
-        const int64_t qi = qw + 16 * qt + row;
-        if (qi >= p.n_q) continue;
+    // ---- output: O[q][c] = O^T / l
+    const float lt = halves_sum(lsum);
+    if (qi < p.n_q) {
         const float r = 1.f / lt;
-        uint16_t *dst = p.out + ((static_cast<int64_t>(b) * p.heads_q + hq) * p.n_q + qi) * kDim;
+        uint16_t *dst = p.out + ((static_cast<int64_t>(b) * p.heads_q + hq) * p.n_q + qi) * kDim + 4 * h;
 #pragma unroll
-        for (int ct = 0; ct < 8; ++ct) {
-            float o[4];
+        for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                o[i] = acc[ct][qt][i] * r;
-                bad |= !finite(o[i]);
+            for (int c = 0; c < 4; ++c) {
+                float o[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    o[i] = acc[ct][4 * c + i] * r;
+                    bad |= !finite(o[i]);
+                }
+                const uint32_t w0 = static_cast<uint32_t>(Elem<DT>::store(o[0])) | (static_cast<uint32_t>(Elem<DT>::store(o[1])) << 16);
+                const uint32_t w1 = static_cast<uint32_t>(Elem<DT>::store(o[2])) | (static_cast<uint32_t>(Elem<DT>::store(o[3])) << 16);
+                *reinterpret_cast<u32x2 *>(dst + 32 * ct + 8 * c) = u32x2{w0, w1};
             }
-            const uint32_t w0 = static_cast<uint32_t>(Elem<DT>::store(o[0])) | (static_cast<uint32_t>(Elem<DT>::store(o[1])) << 16);
-            const uint32_t w1 = static_cast<uint32_t>(Elem<DT>::store(o[2])) | (static_cast<uint32_t>(Elem<DT>::store(o[3])) << 16);
-            *reinterpret_cast<u32x2 *>(dst + 16 * ct + 4 * g) = u32x2{w0, w1};
-        }
     }
     if (bad) raise_status(p.status, NSN_ST_NONFINITE_OUTPUT);
 }

@@ -150,3 +150,27 @@ def test_prefill_bf16_values_beyond_fp16_range():
     scale = np.ones(200)
     scale[3::11] = 1e6
     run_case(28, 1, 2, 2, [130], 200, 3, torch.bfloat16, chunk_scale=scale, weighted=2.0 ** -8)
+
+
+@pytest.mark.parametrize("bits,dtype", [(3, torch.bfloat16), (5, torch.float16)])
+@pytest.mark.parametrize("lengths,n", [([1, 2, 63], 1), ([64, 65, 127], 31), ([128, 129, 191], 33), ([192, 193, 255], 65),
+                                       ([256, 320, 390], 257)])
+def test_prefill_edges_of_the_block_pipeline(lengths, n, bits, dtype):
+    """0 to 6 packed blocks (the packed-only loop runs from 3 on), with and
+    without a tail block, by chunks around a wave's 32 queries, one block and
+    one workgroup: every prologue, hand-over and last half block."""
+    run_case(40, 3, 2, 1, lengths, n, bits, dtype, precise=min(lengths) < 64)
+
+
+def test_prefill_repeats_bit_for_bit():
+    """Every read of a product's result waits for it: the same call twice gives
+    the same bits (a maximum read too early moves only the last place)."""
+    rng = np.random.default_rng(41)
+    L, n = [700, 330], 300
+    x = [torch.from_numpy(normal_tokens(rng, (2, 2), 700)).to(DEV) for _ in range(2)]
+    (kk, seq), (vv, _) = (cache.pack_sequences(t, L, tail_dtype=torch.float16) for t in x)
+    q, kc, vc = (torch.from_numpy(rng.standard_normal((2, h, n, 128)).astype(np.float32)).to(DEV, torch.bfloat16)
+                 for h in (4, 2, 2))
+    first = kernels.prefill_attention(q, kk, vv, seq, kc, vc)
+    for _ in range(4):
+        assert torch.equal(first.view(torch.int16), kernels.prefill_attention(q, kk, vv, seq, kc, vc).view(torch.int16))
