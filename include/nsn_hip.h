@@ -302,6 +302,19 @@ typedef struct {
 int nsn_prefill_attention(const nsn_prefill_args *args, nsn_stream_t stream);
 
 /*
+ * The same attention with every tile's context shared by up to n_splits (1 ..
+ * 16) workgroups and merged by a second kernel: for calls with too few tiles
+ * to fill the GPU (one long sequence, a short chunk).  workspace: at least
+ * nsn_prefill_workspace_floats(..., n_splits) floats, 16-byte aligned (not
+ * read with n_splits 1).  nsn_prefill_splits gives the count that pays for a
+ * call whose sequences hold at most max_blocks 64-token blocks (context, tail
+ * and chunk together); any count gives the same result up to rounding.
+ */
+int nsn_prefill_splits(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t n_q, int64_t max_blocks);
+int64_t nsn_prefill_workspace_floats(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t n_q, int n_splits);
+int nsn_prefill_attention_split(const nsn_prefill_args *args, int n_splits, float *workspace, nsn_stream_t stream);
+
+/*
  * Append n new K and V tokens of `rows` = B*Hkv rows to preallocated tails
  * in place: row r, token i of k_new (at (r*new_row_stride + i)*128 elements)
  * goes to token offset + i of row r of k_tail ([rows, tail_cap, 128]); the

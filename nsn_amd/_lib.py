@@ -83,6 +83,9 @@ SIGNATURES = {
     "nsn_attention_workspace_floats": (I64, [I64, I64, I32]),
     "nsn_finite_scan": (I32, [I32, P, P, P, P, P, P]),
     "nsn_prefill_attention": (I32, [ctypes.POINTER(PrefillArgs), P]),
+    "nsn_prefill_attention_split": (I32, [ctypes.POINTER(PrefillArgs), I32, P, P]),
+    "nsn_prefill_splits": (I32, [I64, I64, I64, I64, I64]),
+    "nsn_prefill_workspace_floats": (I64, [I64, I64, I64, I64, I32]),
     "nsn_tail_append": (I32, [P, P, I64, I64, I64, P, P, I64, I64, I32, P]),
     "nsn_tail_append_cast": (I32, [P, P, I32, I64, I64, I64, P, P, I64, I64, I32, P]),
     "nsn_tail_append_to": (I32, [P, P, I64, I64, I64, P, P, I64, P, I32, P, P]),

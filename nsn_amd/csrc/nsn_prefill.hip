@@ -11,8 +11,12 @@
 // here the packed blocks are dequantised tile by tile into LDS and never reach
 // HBM in dense form.
 //
-// Workgroup = 8 waves = 256 consecutive chunk queries of one (b, q-head);
-// each wave owns 32 queries (one MFMA column tile).  Per 64-token block:
+// Workgroup = 8 waves = 256 rows of one (sequence, kv-head), a row being one
+// chunk query of one of the group's q-heads; each wave owns 32 rows (one MFMA
+// column tile).  Tiles run over head ends: with short chunks a block is
+// dequantised for several heads at once (77 queries x 7 heads: 3 tiles a kv-head
+// instead of 7).  Per 64-token
+// block:
 //   1. the raw block (K/V codes, K/V min and scale, K/V decode factors; for
 //      a tail or chunk block its dense K/V rows) is staged into LDS by DMA
 //      two blocks ahead;
@@ -204,6 +208,28 @@ struct PrefillParams {
     uint16_t *out;             // [B, Hq, n_q, 128] DT
     int32_t *status;
     uint16_t *ka, *va;         // append: the K / V tails written (TDT), else null
+    int splits;                // workgroups that share a tile's blocks (context splits)
+    float *part;               // splits > 1: their partials, see Parts
+};
+
+// Context splits.  A grid of few tiles (one long sequence, a short chunk)
+// leaves most CUs idle, so a tile's blocks are then shared by up to kMaxSplits
+// workgroups and a second kernel merges their softmax states.  A split takes
+// at least kSplitBlocks blocks; the workgroups past nblk / kSplitBlocks leave
+// at once, and a tile with one split left writes its output itself.
+// Workspace: per (tile, split) 256 pairs (running maximum, weight sum), then
+// per (tile, split) the unnormalised O^T in register order, [8 waves][16][64
+// lanes] float4.  A weight sum of kDone marks a tile without partials.
+constexpr int kMaxSplits = 16, kSplitBlocks = 8;
+constexpr float kDone = -1.f;
+struct Parts {
+    float2 *ml;
+    float4 *acc;
+    __device__ Parts(float *part, int64_t tiles, int splits, int64_t tile, int split) {
+        const int64_t slot = tile * splits + split;
+        ml = reinterpret_cast<float2 *>(part) + slot * kQTile;
+        acc = reinterpret_cast<float4 *>(part + 2 * tiles * splits * kQTile) + slot * (kQTile * kDim / 4);
+    }
 };
 
 #pragma clang diagnostic push
@@ -443,27 +469,36 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     const int side = __builtin_amdgcn_readfirstlane(tid >> 8);   // (wave-uniform)
     const int rg = side ? (tid & 15) : ((tid >> 4) & 15);
     const int cg = side ? ((tid >> 4) & 15) : (tid & 15);
-    // Grid (q-head, sequence, query tile), tiles last and in reverse: every
-    // workgroup of the last (longest: it sees the most causal chunk blocks)
-    // tile is dispatched before any of the shorter ones, so the short ones
-    // fill the CUs' last rounds.
-    const int hq = blockIdx.x, b = blockIdx.y;
-    const int kvh = hq / p.group;
-    const int64_t q0 = static_cast<int64_t>(gridDim.z - 1 - blockIdx.z) * kQTile;
-    const int64_t qw = q0 + 32 * wave;                     // this wave's first query
+    // The rows of a kv-head are its group's queries, (q-head, query) in memory
+    // order; a tile is 256 of them, whatever heads they belong to.  Grid (tile,
+    // split, sequence, kv-head), tiles slowest and in reverse: the last tile
+    // holds the latest queries, which see the most causal chunk blocks.
+    const int nq = static_cast<int>(p.n_q);              // (< 2^24, checked by the host)
+    const int nrows = p.group * nq;                      // (rows of 256 bytes: fewer than 2^31 fit the memory)
+    const uint32_t hkv = static_cast<uint32_t>(p.heads_kv);
+    const uint32_t per_tile = gridDim.y > 1 ? hkv : static_cast<uint32_t>(p.batch) * hkv;   // (y: sequences, in a huge grid)
+    const uint32_t zs = blockIdx.x / per_tile, rem = blockIdx.x - zs * per_tile;
+    const uint32_t z = zs / static_cast<uint32_t>(p.splits);
+    const int split = static_cast<int>(zs - z * static_cast<uint32_t>(p.splits));
+    const int b = static_cast<int>(rem / hkv + blockIdx.y);
+    const int kvh = static_cast<int>(rem % hkv);
+    const int tiles = (nrows + kQTile - 1) / kQTile;
+    const int q0 = (tiles - 1 - static_cast<int>(z)) * kQTile;
+    const int rw = q0 + 32 * wave;                       // this wave's first row
+    const int r = rw + col;                              // this lane's row,
+    const int qi = r % nq;                               // and its query
     const int64_t seqrow = static_cast<int64_t>(b) * p.heads_kv + kvh;
+    const int64_t row0 = seqrow * p.group * p.n_q;       // row 0 of q and out
 
-    // ---- Q fragments (B operand of S^T = K' Q^T): query qw + l % 32, channels
+    // ---- Q fragments (B operand of S^T = K' Q^T): row rw + l % 32, channels
     // 16*ks + 8*h + chE[e] (fp16: times scale*log2(e)); loaded before the
     // context lengths are needed, so the two round trips overlap
     u32x4 qf[8];
-    const int64_t qi = qw + col;   // this lane's query
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
         float x[8];
-        if (qi < p.n_q) {
-            const uint4 a = *reinterpret_cast<const uint4 *>(
-                p.q + ((static_cast<int64_t>(b) * p.heads_q + hq) * p.n_q + qi) * kDim + 16 * ks + 8 * h);
+        if (r < nrows) {
+            const uint4 a = *reinterpret_cast<const uint4 *>(p.q + (row0 + r) * kDim + 16 * ks + 8 * h);
             const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -478,23 +513,39 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
                        pk<DT>(x[O::chE[4]], x[O::chE[5]]), pk<DT>(x[O::chE[6]], x[O::chE[7]])};
     }
 
+    auto parts = [&]() {
+        return Parts(p.part, static_cast<int64_t>(tiles) * p.batch * p.heads_kv, p.splits,
+                     (static_cast<int64_t>(q0 / kQTile) * p.batch + b) * p.heads_kv + kvh, split);
+    };
     const int64_t T = p.ctx_len[b];
     const int64_t nbk = p.k.blocks ? p.k.blocks[b] : 0;
     const int64_t nbv = p.v.blocks ? p.v.blocks[b] : 0;
     if (nbk != nbv || nbk < 0 || (nbk > 0 && (nbk > p.k.block_cap || nbk > p.v.block_cap)) || T - nbk * kBlockTok < 0 ||
         T - nbk * kBlockTok > p.k.tail_cap || T - nbk * kBlockTok > p.v.tail_cap) {
         if (tid == 0) raise_status(p.status, NSN_ST_CAPACITY);   // inconsistent cache (host checks first)
+        if (p.splits > 1 && tid < kQTile) parts().ml[tid] = float2{-INFINITY, kDone};
         return;
     }
     const int nb = static_cast<int>(nbk), ntail = static_cast<int>(T - nbk * kBlockTok);
-    const int nq = static_cast<int>(p.n_q);                      // (< 2^24: the grid's limit)
-    const int qend = (q0 + kQTile < nq) ? static_cast<int>(q0) + kQTile : nq;   // chunk tokens this workgroup sees
+    // chunk tokens this workgroup sees: up to its last row's query, all of
+    // them where its rows run over the end of a head
+    const int rl = (q0 + kQTile < nrows ? q0 + kQTile : nrows) - 1;
+    const int qend = (rl / nq == q0 / nq) ? rl % nq + 1 : nq;
     const int nt_blk = static_cast<int>((static_cast<int64_t>(ntail) + kBlockTok - 1) / kBlockTok);
     const int nblk = nb + nt_blk + (qend + kBlockTok - 1) / kBlockTok;
-    // append: the workgroup of the last query tile (it stages every chunk
-    // block) of each kv-head's first q-head writes the chunk's K/V to tail
-    // rows ntail .. ntail + n_q - 1 as it fills them; no room: flag, no append
-    const bool app_wg = p.ka && blockIdx.z == 0 && hq % p.group == 0;
+    // this workgroup's blocks [j0, j1)
+    int splits = nblk / kSplitBlocks;
+    splits = splits < 1 ? 1 : (splits < p.splits ? splits : p.splits);
+    if (split >= splits) {
+        if (tid < kQTile) parts().ml[tid] = float2{-INFINITY, 0.f};
+        return;
+    }
+    const int j0 = static_cast<int>(static_cast<int64_t>(nblk) * split / splits);
+    const int j1 = static_cast<int>(static_cast<int64_t>(nblk) * (split + 1) / splits);
+    // append: the workgroups of a kv-head's last tile (they stage every chunk
+    // block) write the chunk's K/V to tail rows ntail .. ntail + n_q - 1 as
+    // they fill them; no room: flag, no append
+    const bool app_wg = p.ka && z == 0;
     const bool app_ok = app_wg && ntail + p.n_q <= p.k.tail_cap && ntail + p.n_q <= p.v.tail_cap;
     if (app_wg && !app_ok && tid == 0) raise_status(p.status, NSN_ST_CAPACITY);
 
@@ -506,7 +557,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     float m_run = -INFINITY;
     float lsum = 0.f;   // sum of the rounded weights of this lane's tokens (half of the query's)
     bool bad = false;
-    const bool live = qw < p.n_q;   // (a wave past the chunk end only helps stage and fill)
+    const bool live = rw < nrows;   // (a wave past the last row only helps stage and fill)
 
     // Block j: packed (j < nb), tail (nb <= j < nb + nt_blk), or chunk; its rows
     // in use and (chunk blocks) the chunk position of its first token.
@@ -606,7 +657,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
         if (!decltype(packed_c)::value) block_rows(j, valid, cpos);
         if (valid < kBlockTok || cpos >= 0) {   // (uniform) partial or causal block
             // allowed tokens of this block: tok < valid and (chunk blocks) tok <= query - cpos
-            const int rel = (cpos >= 0) ? static_cast<int>(qi) - cpos : kBlockTok;
+            const int rel = (cpos >= 0) ? qi - cpos : kBlockTok;
             const int lim = (rel < valid - 1) ? rel : valid - 1;
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
@@ -678,12 +729,12 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     using K_ = std::integral_constant<int, 0>;
     using V_ = std::integral_constant<int, 1>;
 
-    // ---- prologue: raw blocks 0 and 1 staged together (one round trip), K' of block 0 filled
-    stage(F_{}, 0);
-    if (nblk > 1) stage(F_{}, 1);
+    // ---- prologue: the first two raw blocks staged together (one round trip), K' of the first filled
+    stage(F_{}, j0);
+    if (j0 + 1 < j1) stage(F_{}, j0 + 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (side == 0) fill(K_{}, F_{}, 0);
+    if (side == 0) fill(K_{}, F_{}, j0);
     barrier();
 
     // ---- The two waves of a SIMD (w and w + 4) run half a block out of step,
@@ -711,9 +762,9 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
         attend(packed_c, j);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // raw block j + 1
         barrier();
-        if (PACKED || j + 2 < nblk) stage(packed_c, j + 2);
+        if (PACKED || j + 2 < j1) stage(packed_c, j + 2);
         __builtin_amdgcn_s_setprio(3);
-        if (PACKED || j + 1 < nblk) fill(K_{}, packed_c, j + 1);
+        if (PACKED || j + 1 < j1) fill(K_{}, packed_c, j + 1);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(3);
         if (live) output(j);
@@ -725,28 +776,42 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
         fill(V_{}, packed_c, j);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(3);
-        if (live && j > 0) output(j - 1);
+        if (live && j > j0) output(j - 1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         barrier();
-        if (PACKED || j + 2 < nblk) stage(packed_c, j + 2);
+        if (PACKED || j + 2 < j1) stage(packed_c, j + 2);
         attend(packed_c, j);
         barrier();
     };
-    int j = 0;
+    const int jp = nb < j1 ? nb : j1;
+    int j = j0;
     if (side == 0) {
-        for (; j + 2 < nb; ++j) step_k(T_{}, j);
-        for (; j < nblk; ++j) step_k(F_{}, j);
+        for (; j + 2 < jp; ++j) step_k(T_{}, j);
+        for (; j < j1; ++j) step_k(F_{}, j);
     } else {
-        for (; j + 2 < nb; ++j) step_v(T_{}, j);
-        for (; j < nblk; ++j) step_v(F_{}, j);
-        if (live) output(nblk - 1);
+        for (; j + 2 < jp; ++j) step_v(T_{}, j);
+        for (; j < j1; ++j) step_v(F_{}, j);
+        if (live) output(j1 - 1);
     }
 
     // ---- output: O[q][c] = O^T / l
     const float lt = halves_sum(lsum);
-    if (qi < p.n_q) {
-        const float r = 1.f / lt;
-        uint16_t *dst = p.out + ((static_cast<int64_t>(b) * p.heads_q + hq) * p.n_q + qi) * kDim + 4 * h;
+    if (splits > 1) {   // the split's state instead
+        const Parts pt = parts();
+        if (h == 0) pt.ml[32 * wave + col] = float2{m_run, lt};
+        if (!live) return;
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                pt.acc[(wave * 16 + 4 * ct + c) * 64 + l] =
+                    float4{acc[ct][4 * c], acc[ct][4 * c + 1], acc[ct][4 * c + 2], acc[ct][4 * c + 3]};
+        return;
+    }
+    if (p.splits > 1 && tid < kQTile) parts().ml[tid] = float2{-INFINITY, kDone};
+    if (r < nrows) {
+        const float rl = 1.f / lt;
+        uint16_t *dst = p.out + (row0 + r) * kDim + 4 * h;
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
@@ -754,7 +819,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
                 float o[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    o[i] = acc[ct][4 * c + i] * r;
+                    o[i] = acc[ct][4 * c + i] * rl;
                     bad |= !finite(o[i]);
                 }
                 const uint32_t w0 = static_cast<uint32_t>(Elem<DT>::store(o[0])) | (static_cast<uint32_t>(Elem<DT>::store(o[1])) << 16);
@@ -765,12 +830,131 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     if (bad) raise_status(p.status, NSN_ST_NONFINITE_OUTPUT);
 }
 
+// Merge of the context splits: O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s.
+// One workgroup per 32 rows (a wave's tile) of a tile, one wave per 32 channels:
+// lane l holds row l % 32's channels 32*ct + 8*c + 4*(l/32) .. +3 as the
+// attention kernel left them, so every read is 1 KB in a row.
+template <int DT>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
+    const int l = threadIdx.x & 63, ct = threadIdx.x >> 6;
+    const int64_t tile = blockIdx.x >> 3;
+    const int wave = blockIdx.x & 7;
+    const int nrows = p.group * static_cast<int>(p.n_q);
+    const int64_t per_tile = p.batch * p.heads_kv;
+    const int64_t seqrow = tile % per_tile;
+    const int r = static_cast<int>(tile / per_tile) * kQTile + 32 * wave + (l & 31);
+    const int64_t tiles = (nrows + kQTile - 1) / kQTile * per_tile;
+    float m[kMaxSplits], w[kMaxSplits];
+    float M = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s) {
+        m[s] = -INFINITY;
+        w[s] = 0.f;
+        if (s < p.splits) {
+            const float2 v = Parts(p.part, tiles, p.splits, tile, s).ml[32 * wave + (l & 31)];
+            m[s] = v.x;
+            w[s] = v.y;
+            M = fmaxf(M, v.x);
+        }
+    }
+    if (w[0] == kDone || r >= nrows) return;
+    float L = 0.f;
+    float o[4][4] = {};
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s) {
+        if (s < p.splits && m[s] != -INFINITY) {   // (a split that saw no token of the row has no weight)
+            const float a = __builtin_amdgcn_exp2f(m[s] - M);
+            L = __builtin_fmaf(a, w[s], L);
+            const float4 *src = Parts(p.part, tiles, p.splits, tile, s).acc + (wave * 16 + 4 * ct) * 64 + l;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float4 v = src[64 * c];
+                o[c][0] = __builtin_fmaf(a, v.x, o[c][0]);
+                o[c][1] = __builtin_fmaf(a, v.y, o[c][1]);
+                o[c][2] = __builtin_fmaf(a, v.z, o[c][2]);
+                o[c][3] = __builtin_fmaf(a, v.w, o[c][3]);
+            }
+        }
+    }
+    const float rl = 1.f / L;
+    bool bad = false;
+    uint16_t *dst = p.out + (seqrow * nrows + r) * kDim + 32 * ct + 4 * (l >> 5);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        uint16_t e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float x = o[c][i] * rl;
+            bad |= !finite(x);
+            e[i] = Elem<DT>::store(x);
+        }
+        *reinterpret_cast<u32x2 *>(dst + 8 * c) =
+            u32x2{static_cast<uint32_t>(e[0]) | (static_cast<uint32_t>(e[1]) << 16),
+                  static_cast<uint32_t>(e[2]) | (static_cast<uint32_t>(e[3]) << 16)};
+    }
+    if (bad) raise_status(p.status, NSN_ST_NONFINITE_OUTPUT);
+}
+
+// Workgroups' worth of tiles of a call (256 rows of a kv-head each).
+inline int64_t tile_count(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t n_q) {
+    return (heads_q / heads_kv * n_q + kQTile - 1) / kQTile * batch * heads_kv;
+}
+
 }  // namespace prefill
 }  // namespace nsn
 
 using namespace nsn;
 
+extern "C" int64_t nsn_prefill_workspace_floats(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t n_q,
+                                                int n_splits) {
+    using namespace nsn::prefill;
+    if (batch <= 0 || heads_kv <= 0 || heads_q <= 0 || heads_q % heads_kv || n_q <= 0 || n_splits <= 1) return 0;
+    return tile_count(batch, heads_q, heads_kv, n_q) * n_splits * kQTile * (kDim + 2);
+}
+
+// Context splits that pay.  Times in blocks of one workgroup (1.8 us): a
+// workgroup costs 6 before its first block and after its last, a merge 4 plus
+// its partials' traffic (130 KB per tile and split, written and read).
+// Measured without and with the picked count: 1 sequence x 32 heads x 512
+// queries over 32K tokens 892 -> 305 us (4 splits), over 4000 146 -> 74 (4);
+// 7 x 32 x 128 over 16K 447 -> 292 (2); 6 ragged 5-bit sequences x 28 x 77
+// over 190-3100 88 -> 48 (3); 1 x 16 x 100 over 1000 40 -> 31 (2).  From one
+// tile per CU on a split only pays where it fills a half-empty last round
+// (192 tiles: 281 -> 274 with 4), and below 24 blocks of capacity the merge
+// costs what it saves (1 x 16 x 300 over 600: 41 -> 43 us).
+extern "C" int nsn_prefill_splits(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t n_q, int64_t max_blocks) {
+    using namespace nsn::prefill;
+    if (batch <= 0 || heads_kv <= 0 || heads_q <= 0 || heads_q % heads_kv || n_q <= 0) return 1;
+    const int64_t tiles = tile_count(batch, heads_q, heads_kv, n_q);
+    if (max_blocks < 24) return 1;   // (the shortest context that is split)
+    static const int cus = [] {      // every device is a gfx950
+        int dev = 0, n = 0;
+        return hipGetDevice(&dev) == hipSuccess &&
+                       hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0
+                   ? n
+                   : 256;
+    }();
+    if (tiles >= cus) return 1;
+    const double one = 6.0 + static_cast<double>(max_blocks);
+    double best = 0.9 * one;
+    int splits = 1;
+    for (int s = 2; s <= kMaxSplits && 12 * s <= max_blocks; ++s) {
+        const double t = static_cast<double>((tiles * s + cus - 1) / cus) * (6.0 + static_cast<double>(max_blocks) / s) +
+                         4.0 + 0.036 * static_cast<double>(tiles * s);
+        if (t < best) {
+            best = t;
+            splits = s;
+        }
+    }
+    return splits;
+}
+
 extern "C" int nsn_prefill_attention(const nsn_prefill_args *a, nsn_stream_t stream) {
+    return nsn_prefill_attention_split(a, 1, nullptr, stream);
+}
+
+extern "C" int nsn_prefill_attention_split(const nsn_prefill_args *a, int n_splits, float *workspace,
+                                           nsn_stream_t stream) {
     using namespace nsn::prefill;
     if (!a || !a->q || !a->ctx_len || !a->k_chunk || !a->v_chunk || !a->out) return NSN_EINVAL;
     if (a->batch <= 0 || a->heads_kv <= 0 || a->heads_q % a->heads_kv || a->n_q < 0) return NSN_EINVAL;
@@ -801,7 +985,11 @@ extern "C" int nsn_prefill_attention(const nsn_prefill_args *a, nsn_stream_t str
         if (reinterpret_cast<uintptr_t>(ptr) & 15u) return NSN_EINVAL;
     const int64_t qt = (a->n_q + kQTile - 1) / kQTile;
     if (qt > 65535 || a->heads_q > 0x7fffffff || a->batch > 65535) return NSN_EINVAL;
+    if (n_splits < 1 || n_splits > kMaxSplits) return NSN_EINVAL;
+    if (n_splits > 1 && (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u))) return NSN_EINVAL;
     PrefillParams p{};
+    p.splits = n_splits;
+    p.part = workspace;
     p.q = static_cast<const uint16_t *>(a->q);
     p.batch = a->batch;
     p.heads_q = a->heads_q;
@@ -824,7 +1012,13 @@ extern "C" int nsn_prefill_attention(const nsn_prefill_args *a, nsn_stream_t str
         p.ka = static_cast<uint16_t *>(const_cast<void *>(a->k.tail));
         p.va = static_cast<uint16_t *>(const_cast<void *>(a->v.tail));
     }
-    const dim3 grid(static_cast<unsigned>(a->heads_q), static_cast<unsigned>(a->batch), static_cast<unsigned>(qt));
+    // one workgroup per 256 rows of a kv-head (rows: the queries of its group)
+    const int64_t tiles = (p.group * a->n_q + kQTile - 1) / kQTile * n_splits;
+    const int64_t wgs = tiles * a->batch * a->heads_kv;
+    constexpr int64_t kMaxGrid = 1 << 22;     // workgroups of one grid dimension (2^31 threads)
+    if (tiles * a->heads_kv > kMaxGrid) return NSN_EINVAL;   // (more rows than memory holds)
+    const dim3 grid = wgs <= kMaxGrid ? dim3(static_cast<unsigned>(wgs))
+                                      : dim3(static_cast<unsigned>(tiles * a->heads_kv), static_cast<unsigned>(a->batch));
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const bool bf = a->dtype == NSN_DTYPE_BF16;
 #define NSN_PREFILL_LAUNCH(B_, D_, L_)                                                                              \
@@ -843,5 +1037,11 @@ extern "C" int nsn_prefill_attention(const nsn_prefill_args *a, nsn_stream_t str
         else NSN_PREFILL_LAUNCH(5, NSN_DTYPE_F16, false);
     }
 #undef NSN_PREFILL_LAUNCH
+    if (n_splits > 1) {
+        if (hipGetLastError() != hipSuccess) return NSN_ELAUNCH;
+        const dim3 mgrid(static_cast<unsigned>(8 * (wgs / n_splits)));   // (8 per tile; < 2^25: the grid's limit)
+        if (bf) hipLaunchKernelGGL(prefill_merge_kernel<NSN_DTYPE_BF16>, mgrid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL(prefill_merge_kernel<NSN_DTYPE_F16>, mgrid, dim3(256), 0, st, p);
+    }
     return hipGetLastError() == hipSuccess ? NSN_OK : NSN_ELAUNCH;
 }

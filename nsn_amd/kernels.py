@@ -77,24 +77,25 @@ class PackedKV:
         return s
 
     def validate(self, batch, heads):
-        if self.codes is not None:
-            nbytes = BLOCK * DIM * self.bits // 8
-            require(self.codes.dtype == torch.uint8 and self.codes.is_contiguous() and self.codes.ndim == 4
-                    and tuple(self.codes.shape[:2]) == (batch, heads) and self.codes.shape[3] == nbytes,
-                    "Packed codes layout")
-            cap = self.codes.shape[2]
-            for t, last in ((self.norm, BLOCK), (self.min, DIM), (self.scale, DIM)):
-                require(t.dtype == torch.float16 and t.is_contiguous() and t.numel() == batch * heads * cap * last,
-                        "Packed metadata layout")
-            require(self.blocks is not None and self.blocks.dtype == torch.int32 and self.blocks.numel() == batch,
+        # (each shape is read once: this runs on every attention call)
+        codes, tail, f16 = self.codes, self.tail, torch.float16
+        if codes is not None:
+            shape = codes.shape
+            require(codes.dtype == torch.uint8 and codes.is_contiguous() and len(shape) == 4 and shape[0] == batch
+                    and shape[1] == heads and shape[3] == BLOCK * DIM * self.bits // 8, "Packed codes layout")
+            n = batch * heads * shape[2]
+            norm, mn, sc, f, blocks = self.norm, self.min, self.scale, self.factor, self.blocks
+            require(norm.dtype == f16 and mn.dtype == f16 and sc.dtype == f16 and norm.numel() == n * BLOCK
+                    and mn.numel() == n * DIM and sc.numel() == n * DIM and norm.is_contiguous()
+                    and mn.is_contiguous() and sc.is_contiguous(), "Packed metadata layout")
+            require(blocks is not None and blocks.dtype == torch.int32 and blocks.numel() == batch,
                     "Packed block counts")
-            if self.factor is not None:
-                require(self.factor.dtype == torch.float32 and self.factor.is_contiguous()
-                        and self.factor.numel() == batch * heads * cap * BLOCK, "Decode factor layout")
-        if self.tail is not None:
-            require(self.tail.dtype in (torch.float16, torch.bfloat16) and self.tail.is_contiguous()
-                    and self.tail.ndim == 4 and tuple(self.tail.shape[:2]) == (batch, heads)
-                    and self.tail.shape[3] == DIM, "Tail shape/type")
+            require(f is None or (f.dtype == torch.float32 and f.is_contiguous() and f.numel() == n * BLOCK),
+                    "Decode factor layout")
+        if tail is not None:
+            shape = tail.shape
+            require(tail.dtype in (f16, torch.bfloat16) and tail.is_contiguous() and len(shape) == 4
+                    and shape[0] == batch and shape[1] == heads and shape[3] == DIM, "Tail shape/type")
 
 
 def workspace_floats(batch, heads_q, n_splits):
@@ -302,13 +303,14 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
     the first queries attend a handful of tokens.
     """
     _dev.require_gpu(q, k_chunk, v_chunk, ctx_len)
-    require(q.ndim == 4 and q.shape[3] == DIM and q.is_contiguous(), "Query shape/type")
-    B, Hq, n, _ = q.shape
-    require(q.dtype in (torch.float16, torch.bfloat16), "Prefill dtype (fp16 or bf16)")
-    require(k_chunk.dtype == q.dtype and v_chunk.dtype == q.dtype and k_chunk.shape == v_chunk.shape
-            and k_chunk.ndim == 4 and k_chunk.shape[0] == B and k_chunk.shape[2] == n and k_chunk.shape[3] == DIM
+    qshape, cshape, qdt = q.shape, k_chunk.shape, q.dtype
+    require(len(qshape) == 4 and qshape[3] == DIM and q.is_contiguous(), "Query shape/type")
+    B, Hq, n, _ = qshape
+    require(qdt in (torch.float16, torch.bfloat16), "Prefill dtype (fp16 or bf16)")
+    require(k_chunk.dtype == qdt and v_chunk.dtype == qdt and cshape == v_chunk.shape
+            and len(cshape) == 4 and cshape[0] == B and cshape[2] == n and cshape[3] == DIM
             and k_chunk.is_contiguous() and v_chunk.is_contiguous(), "Chunk K/V shape/type")
-    Hkv = k_chunk.shape[1]
+    Hkv = cshape[1]
     require(Hq % Hkv == 0, "GQA group")
     require(ctx_len.dtype == torch.int32 and ctx_len.numel() == B and ctx_len.is_cuda, "Context lengths")
     a = _lib.PrefillArgs()
@@ -361,8 +363,15 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
     a.status = st.data_ptr()
     a.append = 1 if append else 0
     a.precise_weights = 1 if (k is None if precise_weights is None else precise_weights) else 0
-    rc = _lib.lib().nsn_prefill_attention(a, _dev.stream())
-    _lib.check(rc, "nsn_prefill_attention")
+    # few tiles (one long sequence, a short chunk): split the context too.  The
+    # lengths stay on the device, so the capacity bounds them here; the kernel
+    # uses no more splits than the actual length pays for.
+    lib = _lib.lib()
+    splits, ws = lib.nsn_prefill_splits(B, Hq, Hkv, n, a.k.block_cap + (a.k.tail_cap + n) // BLOCK + 2), None
+    if splits > 1:
+        ws = torch.empty(lib.nsn_prefill_workspace_floats(B, Hq, Hkv, n, splits), dtype=torch.float32, device=q.device)
+    rc = lib.nsn_prefill_attention_split(a, splits, ws if ws is None else ws.data_ptr(), _dev.stream())
+    _lib.check(rc, "nsn_prefill_attention_split")
     if check and status is None:
         s = _dev.read_status(st)
         if s & _lib.ST_CAPACITY:

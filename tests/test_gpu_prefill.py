@@ -162,6 +162,50 @@ def test_prefill_edges_of_the_block_pipeline(lengths, n, bits, dtype):
     run_case(40, 3, 2, 1, lengths, n, bits, dtype, precise=min(lengths) < 64)
 
 
+@pytest.mark.parametrize("Hq,Hkv,n", [(7, 1, 1), (7, 1, 37), (6, 2, 85), (6, 2, 86), (10, 2, 256), (3, 1, 300)])
+def test_prefill_tiles_across_heads(Hq, Hkv, n):
+    """A tile's 256 rows run over the ends of a group's heads: several whole
+    heads a tile, 3 x 85 rows (one short of it) and 3 x 86 (two over), a head
+    a tile, and heads that begin and end inside one; causal inside the chunk."""
+    run_case(42, 2, Hq, Hkv, [200, 70], n, 3, torch.float16)
+
+
+@pytest.mark.parametrize("dtype,bits", [(torch.bfloat16, 3), (torch.float16, 5)])
+@pytest.mark.parametrize("splits,Hq,n", [(2, 4, 70), (3, 2, 1), (5, 4, 300), (16, 2, 33)])
+def test_prefill_context_splits(monkeypatch, splits, Hq, n, dtype, bits):
+    """The tiles' blocks shared by several workgroups and merged: contexts too
+    short to split (one of 300 tokens writes its output itself), 17 blocks (two
+    splits) and 40 (up to five), chunk blocks masked for the first rows of a
+    split, rows past the last, and more splits asked than the blocks allow."""
+    monkeypatch.setattr(kernels._lib.lib(), "nsn_prefill_splits", lambda *a: splits)
+    run_case(43, 3, Hq, 2, [300, 1050, 2500], n, bits, dtype)
+
+
+def test_prefill_context_splits_append(monkeypatch):
+    """The splits of the last tile append the chunk between them: tails and
+    status as without splits, output within one rounding of it."""
+    rng = np.random.default_rng(44)
+    x = [torch.from_numpy(normal_tokens(rng, (2, 2), 2000)).to(DEV) for _ in range(2)]
+    q, kc, vc = (torch.from_numpy(normal_tokens(rng, (2, h), 90)).to(DEV) for h in (4, 2, 2))
+    got = []
+    for splits in (1, 4):
+        monkeypatch.setattr(kernels._lib.lib(), "nsn_prefill_splits", lambda *a: splits)
+        sides = []
+        for t in x:
+            kv, seq = cache.pack_sequences(t, [2000, 700])
+            room = torch.zeros((2, 2, 192, 128), dtype=torch.float16, device=DEV)
+            room[:, :, :kv.tail.shape[2]] = kv.tail
+            kv.tail = room
+            sides.append(kv)
+        out = kernels.prefill_attention(q, sides[0], sides[1], seq, kc, vc, append=True)
+        got.append((out, sides[0].tail, sides[1].tail))
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    d = (got[0][0].float() - got[1][0].float()).abs()
+    # fp16 outputs of the same sums in another order, with fp16 weights whose scale moves with the split's maximum
+    assert bool((d <= 2.0 ** -10 * got[0][0].float().abs() + 2.0 ** -10).all())
+
+
 def test_prefill_repeats_bit_for_bit():
     """Every read of a product's result waits for it: the same call twice gives
     the same bits (a maximum read too early moves only the last place)."""

@@ -223,3 +223,20 @@ def test_integration_binding_stubs_match_the_bindings():
         assert ctypes.sizeof(doc_st) == ctypes.sizeof(pkg_st), name
         for f, _ in doc_st._fields_:
             assert getattr(doc_st, f).offset == getattr(pkg_st, f).offset, (name, f)
+
+
+def test_prefill_split_rule():
+    """Context splits: none from one tile per CU on or for short contexts, at
+    most 16, never below 12 blocks each; the workspace holds every tile's
+    partials (256 rows of a pair and 128 channels per split)."""
+    from nsn_amd import _lib
+    lib = _lib.lib()
+    for B, Hq, Hkv, n, blocks in [(1, 32, 8, 512, 521), (6, 28, 4, 77, 47), (32, 16, 16, 512, 140), (1, 1, 1, 1, 23),
+                                  (1, 1, 1, 1, 100000), (7, 40, 8, 33, 300), (255, 1, 1, 1, 30), (256, 1, 1, 1, 9999)]:
+        tiles = -(-Hq // Hkv * n // 256) * B * Hkv
+        s = lib.nsn_prefill_splits(B, Hq, Hkv, n, blocks)
+        assert 1 <= s <= 16 and (s == 1 or (tiles < 256 and 12 * s <= blocks))
+        assert lib.nsn_prefill_workspace_floats(B, Hq, Hkv, n, s) == (0 if s == 1 else tiles * s * 256 * 130)
+    assert lib.nsn_prefill_splits(1, 32, 8, 512, 521) > 1 and lib.nsn_prefill_splits(1, 3, 2, 512, 521) == 1
+    pa = _lib.PrefillArgs()
+    assert lib.nsn_prefill_attention_split(pa, 2, None, None) == _lib.NSN_EINVAL
