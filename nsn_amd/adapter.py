@@ -374,8 +374,8 @@ class PackedKVCache(Cache):
         return out
 
     def _workspace(self, L):
-        _, n = kernels.default_split(self.batch, self.heads, L)
-        need = kernels.workspace_floats(self.batch, self.heads_q, max(2, n))
+        _, n = kernels.decode_split(self.batch, self.heads, L, "fast")
+        need = kernels.workspace_floats(self.batch, self.heads_q, n)
         if self._ws is None or self._ws.numel() < need:
             self._ws = torch.empty(max(need, 2 * (0 if self._ws is None else self._ws.numel())),
                                    dtype=torch.float32, device=self.store.device)

@@ -112,6 +112,29 @@ def default_split(batch, heads_kv, max_len, target_units=4096, min_split=256):
     return max(BLOCK, split), max(1, math.ceil(max_len / max(BLOCK, split)))
 
 
+def decode_split(batch, heads_kv, max_len, kernel):
+    """(split_tokens, n_splits) of a decode call that names none: default_split,
+    cut finer while the call is too small to fill the GPU with it.
+
+    A short context is bound by the blocks one wave walks in series, so it is
+    spread over up to 2048 waves (the fast kernel's resident ones; 640
+    workgroups of the exact-order kernel, a little over two per CU), in up to
+    128 splits (more make the merge longer than they save).  Measured, 256
+    tokens a split against this rule: fast 1 x 16 kv-heads x 1023 tokens 20.0
+    -> 11.4 us, 5 x 4 x 6500 24.0 -> 18.3, 64 x 8 x 500 29.5 -> 18.4, 1 x 8 x
+    32000 23.7 -> 22.6 (64 tokens: 24.4); exact-order 1 x 16 x 1023 49.5 ->
+    17.5, 1 x 8 x 4133 55.7 -> 30.6, 1 x 8 x 16000 70.2 both ways (64 tokens:
+    81.6).  The fast kernel takes one slot more than there are splits: its
+    blocks per wave are bounded by blocks / (slots - 1).
+    """
+    split, n = default_split(batch, heads_kv, max_len)
+    fine = max(1, min(128, (2048 if kernel == "fast" else 640) // max(1, batch * heads_kv)))
+    finer = max(BLOCK, math.ceil(max_len / fine / BLOCK) * BLOCK)
+    if finer < split:
+        split, n = finer, math.ceil(max_len / finer) + (1 if kernel == "fast" else 0)
+    return split, max(2, n) if kernel == "fast" else n
+
+
 def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=None, scores=None,
                      kernel="reference", kv_round_dtype=None, split_tokens=None, out_dtype=torch.bfloat16,
                      scale=SCALE, status=None, check=True, workspace=None, out=None, ctx=None, merge=True,
@@ -145,7 +168,9 @@ def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=
     if max_seq_len is None:
         max_seq_len = int(seq_len.max().item())
     if split_tokens is None:
-        split_tokens, n_splits = default_split(B, Hkv, max_seq_len)
+        split_tokens, n_splits = decode_split(B, Hkv, max_seq_len, kernel)
+        if static_workspace and workspace_floats(B, Hq, n_splits) > _lib.STATIC_SCRATCH_FLOATS:
+            split_tokens, n_splits = default_split(B, Hkv, max_seq_len)   # (fewer slots: what the scratch holds)
     else:
         n_splits = max(1, math.ceil(max_seq_len / split_tokens))
     if kernel == "fast":

@@ -118,6 +118,23 @@ def test_default_split_covers_context():
         assert split % 64 == 0 and split * n >= L and split * (n - 1) < L
 
 
+def test_decode_split_covers_context_and_bounds_its_slots():
+    """The splits of a call that names none: whole blocks, the context covered,
+    never coarser than default_split, at most 128 finer ones (plus the fast
+    kernel's spare slot), and the fast kernel's slots enough for the blocks a
+    wave takes."""
+    for kernel in ("fast", "reference"):
+        for B, H, L in [(1, 1, 1), (1, 16, 1023), (1, 8, 4133), (1, 8, 32000), (5, 4, 6500), (64, 8, 500), (16, 8, 32768),
+                        (64, 4, 8192), (1, 1, 65), (2048, 1, 4000), (1, 1, 1 << 20)]:
+            base, nb = kernels.default_split(B, H, L)
+            split, n = kernels.decode_split(B, H, L, kernel)
+            assert split % 64 == 0 and split * n >= L and split <= base
+            assert n <= max(nb, 129, 2)
+            if split < base and kernel == "fast":
+                blocks = -(-L // 64)
+                assert -(-blocks // (n - 1)) <= split // 64     # blocks of a wave: what the split asks for
+
+
 def _cpu_fixture(kind):
     """The reference's negative fixtures that fail structural checks (loop_kv_vf01_contract.py:98-120)."""
     a = gi.vf01_fixture(64, 65, "mixed_codes")
