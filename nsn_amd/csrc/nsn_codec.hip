@@ -104,49 +104,6 @@ __device__ __forceinline__ void pack32(const uint32_t (&c)[32], uint32_t (&w)[BI
     }
 }
 
-template <int BITS>
-__device__ __forceinline__ void unpack32(const uint32_t (&w)[BITS], uint32_t (&c)[32]) {
-    constexpr uint32_t mask = (1u << BITS) - 1u;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        const int pos = i * BITS, d = pos >> 5, sh = pos & 31;
-        uint32_t v = w[d] >> sh;
-        if (sh + BITS > 32) v |= w[d + 1] << (32 - sh);
-        c[i] = v & mask;
-    }
-}
-
-// Decode factors f_t = n_t / max(|d_t|, 1e-12) with d_t = m + s*q (fp16 metadata
-// as fp32, unfused multiply/add, torch's 8-lane norm order) for the 64 rows of
-// a block whose u8 codes are in LDS.  f_t * d_t is the row nsn_decode returns
-// (up to the final rounding), so the decode kernels can renormalise a packed
-// token with one multiply.  Writes f_t for t = tid/4 from lanes tid%4 == 0.
-__device__ __forceinline__ void block_factors_lds(const uint8_t *codes_s, const float *m16f, const float *s16f,
-                                                  const float *n16f, float *factors) {
-    const int tid = threadIdx.x;
-    const int r = tid >> 2, jp = (tid & 3) * 2;
-    const uint8_t *cr = codes_s + r * kDim;
-    float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int c = 8 * k + jp;
-        const float p0 = s16f[c] * static_cast<float>(cr[c]);
-        const float p1 = s16f[c + 1] * static_cast<float>(cr[c + 1]);
-        const float d0 = m16f[c] + p0, d1 = m16f[c + 1] + p1;
-        a0 = __builtin_fmaf(d0, d0, a0);
-        a1 = __builtin_fmaf(d1, d1, a1);
-    }
-    const float b0 = __shfl_down(a0, 1), b1 = __shfl_down(a1, 1);
-    const float c0 = __shfl_down(a0, 2), c1 = __shfl_down(a1, 2);
-    const float d0 = __shfl_down(a0, 3), d1 = __shfl_down(a1, 3);
-    if ((tid & 3) == 0) {
-        const float acc[8] = {a0, a1, b0, b1, c0, c1, d0, d1};
-        const float den = clamp_eps(sqrt_rn(lane8_sum(acc)));
-        const float n = n16f[r];
-        factors[r] = (n == 0.f) ? 0.f : div_by_recip(n, recip_rn(den));
-    }
-}
-
 constexpr float kRoundMagic = 12582912.f;   // 1.5 * 2^23: q + this rounds q half-even into the low mantissa bits
 
 typedef _Float16 enc_h2 __attribute__((ext_vector_type(2)));
@@ -660,12 +617,15 @@ struct RestoreParams {
     int32_t *status;
 };
 
-template <int BITS, int OUT_DT, int TAIL_DT>
+// STREAM: an output past the L2s' 32 MB is stored with the non-temporal hint
+// (266 MB of bf16: 77.0 -> 70.8 us); a smaller one stays in them for its reader.
+template <int BITS, int OUT_DT, int TAIL_DT, bool STREAM>
 __global__ __launch_bounds__(256) void restore_kernel(RestoreParams p) {
     using TO = typename Elem<OUT_DT>::T;
-    __shared__ float m_s[kDim], s_s[kDim], n_s[kBlockTok];
+    __shared__ __align__(16) float2 sm_s[kDim];
+    __shared__ float n_s[kBlockTok];
     __shared__ double rden_s[kBlockTok];
-    __shared__ uint32_t codes_s[kBlockTok * kDim / 4];
+    __shared__ __align__(8) uint8_t codes_s[kBlockTok * kCodePitch];
 
     const int tid = threadIdx.x;
     const int64_t o = blockIdx.x / p.tiles_per_outer;
@@ -699,78 +659,56 @@ __global__ __launch_bounds__(256) void restore_kernel(RestoreParams p) {
 
     const int64_t ib = o * p.in_outer_blocks + i;
     if (tid < kDim) {
-        m_s[tid] = f16_bits_to_f32(p.mins[ib * kDim + tid]);
-        s_s[tid] = f16_bits_to_f32(p.scales[ib * kDim + tid]);
+        sm_s[tid] = make_float2(f16_bits_to_f32(p.scales[ib * kDim + tid]), f16_bits_to_f32(p.mins[ib * kDim + tid]));
     } else if (tid < kDim + kBlockTok) {
         n_s[tid - kDim] = f16_bits_to_f32(p.norms[ib * kBlockTok + tid - kDim]);
     }
-    {
-        const int g = tid;
+    if (p.codes_unpacked) {
+        const uint4 *src = reinterpret_cast<const uint4 *>(p.codes + ib * (kBlockTok * kDim)) + 2 * tid;
+        const uint4 a = src[0], b = src[1];
+        const uint32_t c4[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        put_codes(codes_s, tid, c4);
+    } else {
         uint32_t c4[8];
-        if (p.codes_unpacked) {
-            const uint4 *src = reinterpret_cast<const uint4 *>(p.codes + ib * (kBlockTok * kDim)) + 2 * g;
-            const uint4 a = src[0], b = src[1];
-            c4[0] = a.x; c4[1] = a.y; c4[2] = a.z; c4[3] = a.w;
-            c4[4] = b.x; c4[5] = b.y; c4[6] = b.z; c4[7] = b.w;
-        } else {
-            const uint32_t *src = reinterpret_cast<const uint32_t *>(p.codes + ib * packed_block_bytes(BITS)) + g * BITS;
-            uint32_t w[BITS];
-#pragma unroll
-            for (int k = 0; k < BITS; ++k) w[k] = src[k];
-            uint32_t c[32];
-            unpack32<BITS>(w, c);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) c4[k] = c[4 * k] | (c[4 * k + 1] << 8) | (c[4 * k + 2] << 16) | (c[4 * k + 3] << 24);
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) codes_s[g * 8 + k] = c4[k];
+        unpack_bytes<BITS>(p.codes + ib * packed_block_bytes(BITS), tid, c4);
+        put_codes(codes_s, tid, c4);
     }
     __syncthreads();
-
-    // norm of d = m + s*q in torch's 8-lane order (rows are contiguous)
     {
-        const int r = tid >> 2, jp = (tid & 3) * 2;
-        const uint8_t *cr = reinterpret_cast<const uint8_t *>(codes_s) + r * kDim;
-        float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int c = 8 * k + jp;
-            const float p0 = s_s[c] * static_cast<float>(cr[c]);
-            const float p1 = s_s[c + 1] * static_cast<float>(cr[c + 1]);
-            const float d0 = m_s[c] + p0, d1 = m_s[c + 1] + p1;
-            a0 = __builtin_fmaf(d0, d0, a0);
-            a1 = __builtin_fmaf(d1, d1, a1);
-        }
-        const float b0 = __shfl_down(a0, 1), b1 = __shfl_down(a1, 1);
-        const float c0 = __shfl_down(a0, 2), c1 = __shfl_down(a1, 2);
-        const float d0 = __shfl_down(a0, 3), d1 = __shfl_down(a1, 3);
-        if ((tid & 3) == 0) {
-            const float acc[8] = {a0, a1, b0, b1, c0, c1, d0, d1};
-            rden_s[r] = recip_rn(clamp_eps(sqrt_rn(lane8_sum(acc))));
-        }
+        const float nrm = block_row_norm(codes_s, sm_s);
+        if ((tid & 3) == 0) rden_s[tid >> 2] = recip_rn(clamp_eps(nrm));
     }
     __syncthreads();
 
+    float sc[8], mn[8];
+    load_channels(sm_s, cg, sc, mn);
+    uint32_t top = 0;   // a nonfinite 16-bit output's exponent carries here
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int r = r0 + 16 * j;
-        const uint8_t *cr = reinterpret_cast<const uint8_t *>(codes_s) + r * kDim;
+        const uint2 c8 = *reinterpret_cast<const uint2 *>(codes_s + r * kCodePitch + 8 * cg);
         const float n = n_s[r];
         const double rd = rden_s[r];
         float y[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int c = 8 * cg + e;
-            const float prod = s_s[c] * static_cast<float>(cr[c]);
-            const float d = m_s[c] + prod;
-            const float val = n * div_by_recip(d, rd);
-            y[e] = (n == 0.f) ? 0.f : val;
-            y[e] = Elem<OUT_DT>::load(Elem<OUT_DT>::store(y[e]));
-            bad |= !finite(y[e]);
+        for (int e = 0; e < 8; ++e) y[e] = restore_value(e < 4 ? c8.x : c8.y, e & 3, sc[e], mn[e], n, rd);
+        TO *dst = out + (i * kBlockTok + r) * kDim + 8 * cg;
+        if constexpr (OUT_DT == NSN_DTYPE_F32) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bad |= !finite(y[e]);
+            store_row8<OUT_DT>(dst, y);
+        } else {
+            enc_u4 w;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                w[k] = pack16<OUT_DT>(y[2 * k], y[2 * k + 1]);
+                top |= nonfinite16<OUT_DT>(w[k]);
+            }
+            if constexpr (STREAM) __builtin_nontemporal_store(w, reinterpret_cast<enc_u4 *>(dst));
+            else *reinterpret_cast<enc_u4 *>(dst) = w;
         }
-        store_row8<OUT_DT>(out + (i * kBlockTok + r) * kDim + 8 * cg, y);
     }
-    if (bad) raise_status(p.status, NSN_ST_NONFINITE_RESTORE);
+    if (bad || top) raise_status(p.status, NSN_ST_NONFINITE_RESTORE);
 }
 
 // =====================================================================
@@ -781,33 +719,34 @@ template <int BITS>
 __global__ __launch_bounds__(256) void factor_kernel(const uint8_t *codes, const uint16_t *norms, const uint16_t *mins,
                                                      const uint16_t *scales, int64_t n_blocks, int64_t in_outer_blocks,
                                                      float *factors, int32_t *status) {
-    __shared__ float m_s[kDim], s_s[kDim], n_s[kBlockTok];
-    __shared__ uint32_t codes_s[kBlockTok * kDim / 4];
+    __shared__ __align__(16) float2 sm_s[kDim];
+    __shared__ float n_s[kBlockTok];
+    __shared__ __align__(8) uint8_t codes_s[kBlockTok * kCodePitch];
     const int tid = threadIdx.x;
     const int64_t o = blockIdx.x / n_blocks, i = blockIdx.x - o * n_blocks;
     const int64_t ib = o * in_outer_blocks + i;
     bool bad = false;   // nonfinite metadata: the block's raw inputs fail the finite check
     if (tid < kDim) {
-        m_s[tid] = f16_bits_to_f32(mins[ib * kDim + tid]);
-        s_s[tid] = f16_bits_to_f32(scales[ib * kDim + tid]);
-        bad = !finite(m_s[tid]) || !finite(s_s[tid]);
+        const float2 v = make_float2(f16_bits_to_f32(scales[ib * kDim + tid]), f16_bits_to_f32(mins[ib * kDim + tid]));
+        sm_s[tid] = v;
+        bad = !finite(v.x) || !finite(v.y);
     } else if (tid < kDim + kBlockTok) {
         n_s[tid - kDim] = f16_bits_to_f32(norms[ib * kBlockTok + tid - kDim]);
         bad = !finite(n_s[tid - kDim]);
     }
     if (bad && status) raise_status(status, NSN_ST_NONFINITE_ATTN_INPUT);
-    {
-        const uint32_t *src = reinterpret_cast<const uint32_t *>(codes + ib * packed_block_bytes(BITS)) + tid * BITS;
-        uint32_t w[BITS];
-#pragma unroll
-        for (int k = 0; k < BITS; ++k) w[k] = src[k];
-        uint32_t c[32];
-        unpack32<BITS>(w, c);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) codes_s[tid * 8 + k] = c[4 * k] | (c[4 * k + 1] << 8) | (c[4 * k + 2] << 16) | (c[4 * k + 3] << 24);
-    }
+    uint32_t c4[8];
+    unpack_bytes<BITS>(codes + ib * packed_block_bytes(BITS), tid, c4);
+    put_codes(codes_s, tid, c4);
     __syncthreads();
-    block_factors_lds(reinterpret_cast<const uint8_t *>(codes_s), m_s, s_s, n_s, factors + ib * kBlockTok);
+    // f_t = n_t / max(|d_t|, 1e-12): f_t * d_t is the row nsn_decode returns (up
+    // to the final rounding), so the decode kernels renormalise a packed token
+    // with one multiply
+    const float den = clamp_eps(block_row_norm(codes_s, sm_s));
+    if ((tid & 3) == 0) {
+        const float n = n_s[tid >> 2];
+        factors[ib * kBlockTok + (tid >> 2)] = (n == 0.f) ? 0.f : div_by_recip(n, recip_rn(den));
+    }
 }
 
 // =====================================================================
@@ -874,11 +813,18 @@ void encode_dispatch_bits(int bits, int order, hipStream_t s, const EncodeParams
     else encode_dispatch_order<DT, 5>(order, s, p);
 }
 
+template <int BITS, int OUT_DT, int TAIL_DT>
+void restore_launch(dim3 grid, hipStream_t s, const RestoreParams &p) {
+    const bool stream = OUT_DT != NSN_DTYPE_F32 && static_cast<int64_t>(grid.x) * (kBlockTok * kDim * 2) > (int64_t{32} << 20);
+    if (stream) hipLaunchKernelGGL((restore_kernel<BITS, OUT_DT, TAIL_DT, OUT_DT != NSN_DTYPE_F32>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((restore_kernel<BITS, OUT_DT, TAIL_DT, false>), grid, dim3(256), 0, s, p);
+}
+
 template <int BITS, int OUT_DT>
 void restore_dispatch_tail(int tail_dt, dim3 grid, hipStream_t s, const RestoreParams &p) {
-    if (tail_dt == NSN_DTYPE_F16) hipLaunchKernelGGL((restore_kernel<BITS, OUT_DT, NSN_DTYPE_F16>), grid, dim3(256), 0, s, p);
-    else if (tail_dt == NSN_DTYPE_BF16) hipLaunchKernelGGL((restore_kernel<BITS, OUT_DT, NSN_DTYPE_BF16>), grid, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((restore_kernel<BITS, OUT_DT, NSN_DTYPE_F32>), grid, dim3(256), 0, s, p);
+    if (tail_dt == NSN_DTYPE_F16) restore_launch<BITS, OUT_DT, NSN_DTYPE_F16>(grid, s, p);
+    else if (tail_dt == NSN_DTYPE_BF16) restore_launch<BITS, OUT_DT, NSN_DTYPE_BF16>(grid, s, p);
+    else restore_launch<BITS, OUT_DT, NSN_DTYPE_F32>(grid, s, p);
 }
 
 template <int BITS>

@@ -268,3 +268,22 @@ def test_encode_edge_blocks_vs_oracle(bits):
             assert np.array_equal(u16(g["metas"][1]), m_o.reshape(-1)), (name, dt)
             assert np.array_equal(u16(g["metas"][2]), s_o.reshape(-1)), (name, dt)
             assert np.array_equal(g["codes"].cpu().numpy().reshape(-1), O.pack_codes(q_o, bits)), (name, dt)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bits,blocks,rest", [(3, 2049, 0), (5, 2048, 70), (4, 2047, 64)])
+def test_restore_streamed_outputs(dtype, bits, blocks, rest):
+    """Outputs past 32 MiB (2048 tiles of 16-bit values) take the streaming
+    stores: bit for bit what the same blocks give in small calls, tail tiles included."""
+    g = torch.Generator(device=DEV).manual_seed(bits)
+    x = torch.randn((1, 1, blocks, 64, 128), generator=g, device=DEV).to(torch.float16)
+    p = codec.encode_group(x, 0, bits)
+    codes, metas = p["codes"].reshape(1, blocks, -1), [m.reshape(1, blocks, -1) for m in p["metas"]]
+    tail = None if rest == 0 else torch.randn((1, rest, 128), generator=g, device=DEV).to(torch.float16)
+    got = codec.restore(codes, metas, bits, dtype, tail=tail)
+    view = torch.int32 if dtype == torch.float32 else torch.int16
+    for i in range(0, blocks, 500):
+        part = codec.restore(codes[:, i:i + 500].contiguous(), [m[:, i:i + 500].contiguous() for m in metas], bits, dtype)
+        assert torch.equal(part.view(view), got[:, 64 * i:64 * i + part.shape[1]].contiguous().view(view))
+    if rest:
+        assert torch.equal(got[:, 64 * blocks:].view(view), tail.to(dtype).view(view))
