@@ -60,85 +60,75 @@ __device__ __forceinline__ float load_elem(const void *base, int64_t idx) {
 constexpr int kBadRestore = 1;   // a reconstructed value is nonfinite
 constexpr int kBadInput = 2;     // a raw input (block metadata, tail token) is nonfinite
 
-// Reconstruct packed block `blk` of row `row` (= b*Hkv + kvh) into tile[64][kXP]
-// as fp32 values already rounded to RDT.  Returns kBad* flags.
-template <int BITS, int RDT>
-__device__ int restore_tile(const SideParams &sd, int64_t row, int64_t blk, float *tile, uint32_t *codes_s,
-                             float *m_s, float *s_s, float *n_s, double *rden_s) {
-    constexpr int kXP = kDim + 4;
+// A thread's share of a packed block as it lies in memory: 32 codes and one
+// metadata value (threads 0-127: scale and min of a channel, 128-191: a norm).
+template <int BITS> struct RawBlock {
+    uint32_t w[BITS];
+    uint16_t a, b;
+};
+template <int BITS>
+__device__ __forceinline__ RawBlock<BITS> load_raw(const SideParams &sd, int64_t row, int64_t blk) {
     const int tid = threadIdx.x;
     const int64_t ib = row * sd.block_cap + blk;
+    RawBlock<BITS> r;
+    const uint32_t *src = reinterpret_cast<const uint32_t *>(sd.codes + ib * packed_block_bytes(BITS)) + tid * BITS;
+#pragma unroll
+    for (int k = 0; k < BITS; ++k) r.w[k] = src[k];
+    r.a = r.b = 0;
+    if (tid < kDim) {
+        r.a = sd.scales[ib * kDim + tid];
+        r.b = sd.mins[ib * kDim + tid];
+    } else if (tid < kDim + kBlockTok) {
+        r.a = sd.norms[ib * kBlockTok + tid - kDim];
+    }
+    return r;
+}
+
+// Reconstruct a packed block into tile[64][kXP] as fp32 values already rounded
+// to RDT.  Returns kBad* flags.
+template <int BITS, int RDT>
+__device__ int restore_tile(const RawBlock<BITS> &raw, float *tile, uint8_t *codes_s, float2 *sm_s, float *n_s,
+                            double *rden_s) {
+    constexpr int kXP = kDim + 4;
+    const int tid = threadIdx.x;
     bool bad_in = false;   // the grouped finite check of the metadata, fused here
     if (tid < kDim) {
-        m_s[tid] = f16_bits_to_f32(sd.mins[ib * kDim + tid]);
-        s_s[tid] = f16_bits_to_f32(sd.scales[ib * kDim + tid]);
-        bad_in = !finite(m_s[tid]) || !finite(s_s[tid]);
+        const float2 v = make_float2(f16_bits_to_f32(raw.a), f16_bits_to_f32(raw.b));
+        sm_s[tid] = v;
+        bad_in = !finite(v.x) || !finite(v.y);
     } else if (tid < kDim + kBlockTok) {
-        n_s[tid - kDim] = f16_bits_to_f32(sd.norms[ib * kBlockTok + tid - kDim]);
+        n_s[tid - kDim] = f16_bits_to_f32(raw.a);
         bad_in = !finite(n_s[tid - kDim]);
     }
-    {
-        const uint32_t *src = reinterpret_cast<const uint32_t *>(sd.codes + ib * packed_block_bytes(BITS)) + tid * BITS;
-        uint32_t w[BITS];
-#pragma unroll
-        for (int k = 0; k < BITS; ++k) w[k] = src[k];
-        constexpr uint32_t mask = (1u << BITS) - 1u;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            uint32_t word = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = 4 * k + e, pos = i * BITS, d = pos >> 5, sh = pos & 31;
-                uint32_t v = w[d] >> sh;
-                if (sh + BITS > 32) v |= w[d + 1] << (32 - sh);
-                word |= (v & mask) << (8 * e);
-            }
-            codes_s[tid * 8 + k] = word;
-        }
-    }
+    uint32_t c4[8];
+    unpack_bytes<BITS>(raw.w, c4);
+    put_codes(codes_s, tid, c4);
     __syncthreads();
     {
-        const int r = tid >> 2, jp = (tid & 3) * 2;
-        const uint8_t *cr = reinterpret_cast<const uint8_t *>(codes_s) + r * kDim;
-        float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int c = 8 * k + jp;
-            const float p0 = s_s[c] * static_cast<float>(cr[c]);
-            const float p1 = s_s[c + 1] * static_cast<float>(cr[c + 1]);
-            const float d0 = m_s[c] + p0, d1 = m_s[c + 1] + p1;
-            a0 = __builtin_fmaf(d0, d0, a0);
-            a1 = __builtin_fmaf(d1, d1, a1);
-        }
-        const float b0 = __shfl_down(a0, 1), b1 = __shfl_down(a1, 1);
-        const float c0 = __shfl_down(a0, 2), c1 = __shfl_down(a1, 2);
-        const float d0 = __shfl_down(a0, 3), d1 = __shfl_down(a1, 3);
-        if ((tid & 3) == 0) {
-            const float acc[8] = {a0, a1, b0, b1, c0, c1, d0, d1};
-            rden_s[r] = recip_rn(clamp_eps(sqrt_rn(lane8_sum(acc))));
-        }
+        const float nrm = block_row_norm(codes_s, sm_s);
+        if ((tid & 3) == 0) rden_s[tid >> 2] = recip_rn(clamp_eps(nrm));
     }
     __syncthreads();
     bool bad = false;
     const int cg = tid & 15, r0 = tid >> 4;
+    float sc[8], mn[8];
+    load_channels(sm_s, cg, sc, mn);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int r = r0 + 16 * j;
-        const uint8_t *cr = reinterpret_cast<const uint8_t *>(codes_s) + r * kDim;
+        const uint2 c8 = *reinterpret_cast<const uint2 *>(codes_s + r * kCodePitch + 8 * cg);
         const float n = n_s[r];
         const double rd = rden_s[r];
-        float *dst = tile + r * kXP + 8 * cg;
+        float y[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const int c = 8 * cg + e;
-            const float prod = s_s[c] * static_cast<float>(cr[c]);
-            const float d = m_s[c] + prod;
-            const float val = n * div_by_recip(d, rd);
-            float y = (n == 0.f) ? 0.f : val;
-            y = Elem<RDT>::load(Elem<RDT>::store(y));
-            bad |= !finite(y);
-            dst[e] = y;
+            y[e] = restore_value(e < 4 ? c8.x : c8.y, e & 3, sc[e], mn[e], n, rd);
+            y[e] = Elem<RDT>::load(Elem<RDT>::store(y[e]));
+            bad |= !finite(y[e]);
         }
+        float4 *dst = reinterpret_cast<float4 *>(tile + r * kXP + 8 * cg);
+        dst[0] = make_float4(y[0], y[1], y[2], y[3]);
+        dst[1] = make_float4(y[4], y[5], y[6], y[7]);
     }
     return (bad ? kBadRestore : 0) | (bad_in ? kBadInput : 0);
 }
@@ -170,24 +160,18 @@ __device__ int dense_tile(const SideParams &sd, int64_t row, int64_t t0, int val
     return bad ? kBadInput : 0;
 }
 
-template <int BITS, int RDT, int TDT>
-__device__ int load_tile(const SideParams &sd, int64_t row, int b, int64_t t0, int valid, float *tile,
-                          uint32_t *codes_s, float *m_s, float *s_s, float *n_s, double *rden_s) {
-    const int64_t nb = sd.blocks ? sd.blocks[b] : 0;
-    if (t0 < nb * kBlockTok)
-        return restore_tile<BITS, RDT>(sd, row, t0 / kBlockTok, tile, codes_s, m_s, s_s, n_s, rden_s);
-    return dense_tile<TDT>(sd, row, t0 - nb * kBlockTok, valid, tile);
-}
-
 template <int BITS, int QDT, int RDT, int TDT, bool SCORES>
 __global__ __launch_bounds__(256) void attn_reference_kernel(AttnParams p) {
     constexpr int kXP = kDim + 4;
-    __shared__ float tile[kBlockTok * kXP];
-    __shared__ uint32_t codes_s[kBlockTok * kDim / 4];
-    __shared__ float m_s[kDim], s_s[kDim], n_s[kBlockTok];
+    __shared__ __align__(16) float tile[kBlockTok * kXP];
+    __shared__ __align__(8) uint8_t codes_s[kBlockTok * kCodePitch];
+    __shared__ __align__(16) float2 sm_s[kDim];
+    __shared__ float n_s[kBlockTok];
     __shared__ double rden_s[kBlockTok];
-    __shared__ float q_s[kMaxGroup * kDim];
-    __shared__ float sc_s[kMaxGroup * kBlockTok];
+    // (q as stored: with fp32 copies a workgroup took 56.8 KB, two per CU)
+    using TQ = typename Elem<QDT>::T;
+    __shared__ __align__(16) TQ q_s[kMaxGroup * kDim];
+    __shared__ __align__(16) float sc_s[kMaxGroup * kBlockTok];
     __shared__ float run_m[kMaxGroup], run_l[kMaxGroup], alpha_s[kMaxGroup];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -226,11 +210,22 @@ __global__ __launch_bounds__(256) void attn_reference_kernel(AttnParams p) {
     bool bad_in = false;   // raw inputs: q, block metadata, tail tokens (the fused finite check)
     for (int i = tid; i < G * kDim; i += 256) {
         const int h = i / kDim, c = i - h * kDim;
-        q_s[i] = load_elem<QDT>(p.q, (static_cast<int64_t>(b) * p.heads_q + hq0 + h) * kDim + c);
-        bad_in |= !finite(q_s[i]);
+        q_s[i] = static_cast<const TQ *>(p.q)[(static_cast<int64_t>(b) * p.heads_q + hq0 + h) * kDim + c];
+        bad_in |= !finite(Elem<QDT>::load(q_s[i]));
     }
     if (tid < G) { run_m[tid] = -INFINITY; run_l[tid] = 0.f; }
     bool bad_attn = false, bad_restore = false;
+    // The packed blocks of a tile's two sides are loaded together, and the next
+    // tile's while this one's V is multiplied: one memory round trip a tile
+    // where each side's loads used to wait for the other side's work.
+    const int64_t kpack = (!SCORES && p.k.blocks) ? p.k.blocks[b] * static_cast<int64_t>(kBlockTok) : 0;
+    const int64_t vpack = p.v.blocks ? p.v.blocks[b] * static_cast<int64_t>(kBlockTok) : 0;
+    RawBlock<BITS> kraw, vraw;
+    auto fetch = [&](int64_t t0) {
+        if (t0 < t_end && t0 < kpack) kraw = load_raw<BITS>(p.k, row, t0 / kBlockTok);
+        if (t0 < t_end && t0 < vpack) vraw = load_raw<BITS>(p.v, row, t0 / kBlockTok);
+    };
+    fetch(t_begin);
     __syncthreads();
 
     for (int64_t t0 = t_begin; t0 < t_end; t0 += kBlockTok) {
@@ -249,19 +244,32 @@ __global__ __launch_bounds__(256) void attn_reference_kernel(AttnParams p) {
                 sc_s[i] = s;
             }
         } else {
-            const int fl = load_tile<BITS, RDT, TDT>(p.k, row, b, t0, valid, tile, codes_s, m_s, s_s, n_s, rden_s);
+            const int fl = (t0 < kpack) ? restore_tile<BITS, RDT>(kraw, tile, codes_s, sm_s, n_s, rden_s)
+                                        : dense_tile<TDT>(p.k, row, t0 - kpack, valid, tile);
             bad_restore |= (fl & kBadRestore) != 0;
             bad_in |= (fl & kBadInput) != 0;
             __syncthreads();
             const int r = tid >> 2, qq = tid & 3;
+            float kr[32];   // the thread's quarter row, read once for every head
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const float4 v = *reinterpret_cast<const float4 *>(tile + r * kXP + 32 * qq + 4 * c);
+                kr[4 * c] = v.x; kr[4 * c + 1] = v.y; kr[4 * c + 2] = v.z; kr[4 * c + 3] = v.w;
+            }
+#pragma unroll 4
             for (int h = 0; h < G; ++h) {
                 float part = 0.f;
-                const float *kr = tile + r * kXP + 32 * qq;
-                const float *qh = q_s + h * kDim + 32 * qq;
-#pragma unroll 8
-                for (int c = 0; c < 32; ++c) {
-                    const float prod = kr[c] * qh[c];
-                    part = part + prod;
+                const TQ *qh = q_s + h * kDim + 32 * qq;
+                constexpr int N = 16 / static_cast<int>(sizeof(TQ));   // elements of a 16-byte read
+#pragma unroll
+                for (int c = 0; c < 32; c += N) {
+                    TQ qv[N];
+                    __builtin_memcpy(qv, __builtin_assume_aligned(qh + c, 16), 16);
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        const float prod = kr[c + i] * Elem<QDT>::load(qv[i]);
+                        part = part + prod;
+                    }
                 }
                 const float o1 = __shfl_down(part, 1), o2 = __shfl_down(part, 2), o3 = __shfl_down(part, 3);
                 if (qq == 0) {
@@ -302,10 +310,12 @@ __global__ __launch_bounds__(256) void attn_reference_kernel(AttnParams p) {
         __syncthreads();
         // ---- V tile and P.V ----
         {
-            const int fl = load_tile<BITS, RDT, TDT>(p.v, row, b, t0, valid, tile, codes_s, m_s, s_s, n_s, rden_s);
+            const int fl = (t0 < vpack) ? restore_tile<BITS, RDT>(vraw, tile, codes_s, sm_s, n_s, rden_s)
+                                        : dense_tile<TDT>(p.v, row, t0 - vpack, valid, tile);
             bad_restore |= (fl & kBadRestore) != 0;
             bad_in |= (fl & kBadInput) != 0;
         }
+        fetch(t0 + kBlockTok);
         __syncthreads();
         if (p.trace_v)   // the V rows this block multiplies (row = b * Hkv + kv-head)
             for (int i = tid; i < valid * kDim; i += 256) {
@@ -319,13 +329,24 @@ __global__ __launch_bounds__(256) void attn_reference_kernel(AttnParams p) {
                 const float alpha = alpha_s[h];
                 float a0 = acc[k][0] * alpha, a1 = acc[k][1] * alpha;
                 const float *ph = sc_s + h * kBlockTok;
-                for (int t = 0; t < valid; ++t) {
-                    const float w = ph[t];
-                    const float2 vv = *reinterpret_cast<const float2 *>(tile + t * kXP + 2 * lane);
+                // eight tokens' operands in flight: one at a time, every step of
+                // the sum waited for its own LDS read
+                auto add = [&](float w, float2 vv) {
                     const float p0 = w * vv.x, p1 = w * vv.y;
                     a0 = a0 + p0;
                     a1 = a1 + p1;
+                };
+                auto val = [&](int t) { return *reinterpret_cast<const float2 *>(tile + t * kXP + 2 * lane); };
+                int t = 0;
+                for (; t + 8 <= valid; t += 8) {
+                    float2 vv[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) vv[i] = val(t + i);
+                    const float4 w0 = *reinterpret_cast<const float4 *>(ph + t), w1 = *reinterpret_cast<const float4 *>(ph + t + 4);
+                    add(w0.x, vv[0]); add(w0.y, vv[1]); add(w0.z, vv[2]); add(w0.w, vv[3]);
+                    add(w1.x, vv[4]); add(w1.y, vv[5]); add(w1.z, vv[6]); add(w1.w, vv[7]);
                 }
+                for (; t < valid; ++t) add(ph[t], val(t));
                 acc[k][0] = a0;
                 acc[k][1] = a1;
             }
