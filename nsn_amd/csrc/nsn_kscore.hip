@@ -145,15 +145,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     const int ch0 = grp * CPL;   // the lane's channel block
     float wv[CPL];
     float mx = 0.f, c0p = 0.f;
-    const uint16_t *qrow = p.q + ((b * p.heads_q + hq0 + (h_a < G ? h_a : 0)) * D);
-    const int64_t cbase = b * p.heads_kv * D + static_cast<int64_t>(hkv) * D;
+    // All of the lane's q, step and min values are requested before the first is
+    // used, 16 bytes at a time (any 2-byte alignment); one by one behind the
+    // head test they were a chain of round trips (16 x 32K u8 tokens 137.8 ->
+    // 129.2 us with the uniform tile steps below, 3 x 7.8K 11.5 -> 9.3 us).
+    const uint16_t *qrow = p.q + ((b * p.heads_q + hq0 + (h_a < G ? h_a : 0)) * D) + ch0;
+    const int64_t cbase = b * p.heads_kv * D + static_cast<int64_t>(hkv) * D + ch0;
+    uint4 q4[CPL / 8], s4[CPL / 8], m4[CPL / 8];
+#pragma unroll
+    for (int k = 0; k < CPL / 8; ++k) {
+        __builtin_memcpy(&q4[k], qrow + 8 * k, 16);
+        if constexpr (MODE != MODE_FP16) {
+            __builtin_memcpy(&s4[k], p.steps + cbase + 8 * k, 16);
+            __builtin_memcpy(&m4[k], p.mins + cbase + 8 * k, 16);
+        }
+    }
+    auto half_at = [](const uint4 &v, int e) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        return h2f(static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1))));
+    };
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
-        const float qv = (h_a < G) ? h2f(qrow[ch0 + i]) : 0.f;
+        const float qv = (h_a < G) ? half_at(q4[i / 8], i % 8) : 0.f;
         float w = qv;
         if constexpr (MODE != MODE_FP16) {
-            w = qv * h2f(p.steps[cbase + ch0 + i]);
-            c0p = __builtin_fmaf(qv, h2f(p.mins[cbase + ch0 + i]), c0p);
+            w = qv * half_at(s4[i / 8], i % 8);
+            c0p = __builtin_fmaf(qv, half_at(m4[i / 8], i % 8), c0p);
         }
         wv[i] = w;
         mx = fmaxf(mx, fabsf(w));
@@ -204,15 +221,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
     float *const outB = p.out + (b * p.heads_q + hq0 + hB) * T;
     const bool stA = hA < G, stB = hB < G;
 
-    // ---- tiles: lane loads its token's channel block, PF tiles ahead
+    // ---- tiles: lane loads its token's channel block, PF tiles ahead.  Tile it
+    // is a uniform step from the lane's first token; only the sequence's last
+    // tile can be partial (its lanes past the end read the last token again).
+    const int64_t t_row = it0 * 16 + row;
     const uint8_t *const cl = p.codes + b * T * p.row_bytes + static_cast<int64_t>(hkv) * (D * SH::LANE_BYTES / CPL) +
-                              grp * SH::LANE_BYTES;
-    const uint16_t *const enl = NSN ? p.en + (b * p.heads_kv + hkv) * T : nullptr;
+                              grp * SH::LANE_BYTES + t_row * p.row_bytes;
+    const uint16_t *const enl = NSN ? p.en + (b * p.heads_kv + hkv) * T + t_row : nullptr;
+    const int64_t step = 16 * p.row_bytes;
+    const int last_row = static_cast<int>((T - 1) & 15);   // last row in use of the sequence's last tile
     auto load = [&](int64_t it) {
         Tile<D, MODE, BITS> r;
-        int64_t t = it * 16 + row;
-        t = t < T ? t : T - 1;
-        const uint8_t *src = cl + t * p.row_bytes;
+        const int64_t n = it - it0;
+        const uint8_t *src = cl + n * step;
+        const uint16_t *e = enl + 16 * n;
+        if (it == ntiles_all - 1 && row > last_row) {
+            src -= (row - last_row) * p.row_bytes;
+            e -= row - last_row;
+        }
         if constexpr (NW % 4 == 0) {
 #pragma unroll
             for (int k = 0; k < NW / 4; ++k) {
@@ -223,21 +249,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 
 #pragma unroll
             for (int k = 0; k < NW; ++k) r.w[k] = reinterpret_cast<const uint32_t *>(src)[k];
         }
-        r.en = NSN ? enl[t] : 0u;
+        r.en = NSN ? *e : 0u;
         return r;
     };
+    float *const oA = outA + t_row, *const oB = outB + t_row;
     auto process = [&](const Tile<D, MODE, BITS> &r, int64_t it) {
         u32x4 Bf[NK];
         b_frags<D, MODE, BITS>(r, Bf);
         f32x4 C = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < NK; ++kk) C = mfma(A[kk], Bf[kk], C);
-        const int64_t t = it * 16 + row;
-        if (t < T) {
-            const float f = NSN ? h2f(static_cast<uint16_t>(r.en)) * p.scale : p.scale;
-            if (stA) outA[t] = ((C[0] + C[1]) * kA + c0A) * f;
-            if (stB) outB[t] = ((C[2] + C[3]) * kB + c0B) * f;
-        }
+        const bool in = it < ntiles_all - 1 || row <= last_row;
+        const float f = NSN ? h2f(static_cast<uint16_t>(r.en)) * p.scale : p.scale;
+        if (in && stA) oA[16 * (it - it0)] = ((C[0] + C[1]) * kA + c0A) * f;
+        if (in && stB) oB[16 * (it - it0)] = ((C[2] + C[3]) * kB + c0B) * f;
     };
     Tile<D, MODE, BITS> buf[PF];
 #pragma unroll
@@ -301,9 +326,18 @@ extern "C" int nsn_kscore(const nsn_kscore_args *a, nsn_stream_t stream) {
     if ((reinterpret_cast<uintptr_t>(a->q) & 1u) || (reinterpret_cast<uintptr_t>(a->out) & 3u)) return NSN_EINVAL;
     const int64_t streams = a->batch * a->heads_kv;
     const int64_t tiles = (a->T + 15) / 16;
-    // about 16 waves per CU over 256 CUs, each a contiguous run of tiles
+    // One round of 16 waves per CU over 256 CUs, each a contiguous run of tiles,
+    // while the runs are short; longer ones are cut into at least four rounds
+    // of at least 8 tiles (16 at head_dim 256, whose prologue is twice as long),
+    // so that the CUs and XCDs that run ahead take more of them (16 x 32K
+    // tokens: u8 129.2 -> 122.4 us, 3-bit 73.2 -> 69.8 us; short calls would
+    // lose: 3 x 7.8K tokens in 8-tile runs or finer 9.3 -> 15.7 us).
     int64_t chunk = (streams * tiles + 4095) / 4096;
-    chunk = chunk < 1 ? 1 : (chunk > 64 ? 64 : chunk);
+    const int64_t least = D / 16;
+    if (chunk >= 4 * least) {
+        chunk = (streams * tiles + 16383) / 16384;
+        chunk = chunk < least ? least : (chunk > 64 ? 64 : chunk);
+    }
     const int64_t n_chunks = (tiles + chunk - 1) / chunk;
     const int64_t waves = streams * n_chunks;
     if ((waves + 3) / 4 > 0x7fffffff) return NSN_EINVAL;

@@ -113,3 +113,28 @@ def test_kscore_reference_golden_scores(recipe, bits):
     got = kscore.decode_scores(q, ts, n_q, 8, D).cpu().double().numpy()
     ref = G[key + "scores"].astype(np.float64)
     assert np.abs(got - ref).max() <= REL_MAX * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("fp16", [False, True])
+def test_kscore_short_runs_match_single_sequences(fp16):
+    """A call large enough for four rounds of shorter runs (the last tile of
+    each sequence partial), and queries, steps and minima at 2-byte
+    alignments: bit for bit the scores of one sequence at a time."""
+    B, n_kv, D, n_q, T = 4, 16, 128, 32, 32773
+    g = torch.Generator(device=DEV).manual_seed(5)
+
+    def odd(shape, scale):   # contiguous, 2 bytes past a 16-byte boundary
+        flat = torch.randn(int(np.prod(shape)) + 1, generator=g, device=DEV).mul_(scale).half()
+        return flat[1:].view(shape)
+    q = odd((B, n_q, D), 1.0)
+    if fp16:
+        ts = {"code": torch.randn((B, T, n_kv * D), generator=g, device=DEV, dtype=torch.float16), "is_fp16": True,
+              "is_nsn": False, "T": T}
+    else:
+        ts = {"code": torch.randint(0, 32, (B, T, n_kv * D), generator=g, device=DEV, dtype=torch.uint8), "is_fp16": False,
+              "is_nsn": True, "min": odd((B, n_kv * D), 0.1), "step": odd((B, n_kv * D), 0.02).abs_(),
+              "eff_norm": torch.rand((B, n_kv, T), generator=g, device=DEV).half(), "T": T}
+    got = kscore.decode_scores(q, ts, n_q, n_kv, D)
+    for b in range(B):
+        one = {k: (v[b:b + 1].clone() if torch.is_tensor(v) else v) for k, v in ts.items()}
+        assert torch.equal(got[b:b + 1], kscore.decode_scores(q[b:b + 1].clone(), one, n_q, n_kv, D))
