@@ -58,23 +58,15 @@ class PackedKV:
         return (self.codes if self.codes is not None else self.tail).shape[1]
 
     def side(self):
-        s = _lib.KVSide()
-        if self.codes is not None:
-            s.codes = self.codes.data_ptr()
-            s.norms = self.norm.data_ptr()
-            s.mins = self.min.data_ptr()
-            s.scales = self.scale.data_ptr()
-            if self.factor is not None:
-                s.factors = self.factor.data_ptr()
-            s.blocks = self.blocks.data_ptr()
-            s.block_cap = self.codes.shape[2]
-        if self.tail is not None:
-            s.tail = self.tail.data_ptr()
-            s.tail_dtype = _dev.dtype_code(self.tail.dtype)
-            s.tail_cap = self.tail.shape[2]
-        else:
-            s.tail_dtype = _lib.DTYPE_F16
-        return s
+        # (one constructor call, 1 us: this runs twice on every attention call)
+        codes, tail = self.codes, self.tail
+        tp, tdt, tcap = (None, _lib.DTYPE_F16, 0) if tail is None else \
+            (tail.data_ptr(), _dev.dtype_code(tail.dtype), tail.shape[2])
+        if codes is None:
+            return _lib.KVSide(None, None, None, None, None, None, 0, tp, tdt, tcap)
+        return _lib.KVSide(codes.data_ptr(), self.norm.data_ptr(), self.min.data_ptr(), self.scale.data_ptr(),
+                           None if self.factor is None else self.factor.data_ptr(), self.blocks.data_ptr(),
+                           codes.shape[2], tp, tdt, tcap)
 
     def validate(self, batch, heads):
         # (each shape is read once: this runs on every attention call)
@@ -141,8 +133,9 @@ def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=
     """decode_attention's checks and argument block: (entry point, args,
     status, out, ctx, workspace)."""
     _dev.require_gpu(q, seq_len)
-    require(q.ndim == 3 and q.shape[2] == DIM and q.is_contiguous(), "Query shape/type")
-    B, Hq = q.shape[:2]
+    shape = q.shape
+    require(len(shape) == 3 and shape[2] == DIM and q.is_contiguous(), "Query shape/type")
+    B, Hq, _ = shape
     Hkv = v.heads
     require(Hq % Hkv == 0 and Hq // Hkv <= 16, "GQA group")
     require(seq_len.dtype == torch.int32 and seq_len.numel() == B and seq_len.is_cuda, "Sequence lengths")
@@ -191,31 +184,14 @@ def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=
     if ctx is None:
         ctx = torch.empty((B, Hq, DIM), dtype=torch.float32, device=dev)
     st = status if status is not None else _dev.new_status(dev)
-    a = _lib.AttnArgs()
-    a.q = q.data_ptr()
-    a.q_dtype = _dev.dtype_code(q.dtype)
-    a.batch, a.heads_q, a.heads_kv = B, Hq, Hkv
-    a.scale = scale
-    a.seq_len = seq_len.data_ptr()
-    a.max_seq_len = max_seq_len
-    a.bits = v.bits
-    a.k_mode = _lib.KV_SCORES if scores is not None else _lib.KV_PACKED
-    if scores is None:
-        a.k = k.side()
-    else:
-        a.scores = scores.data_ptr()
-        a.scores_cap = scores.shape[2]
-    a.v = v.side()
-    a.kernel = KERNELS[kernel]
-    a.kv_round_dtype = _dev.dtype_code(kv_round_dtype)
-    a.split_tokens = split_tokens
-    a.n_splits = n_splits
-    a.partials = 0 if static_workspace else workspace.data_ptr()
-    a.ctx = ctx.data_ptr()
-    a.out = out.data_ptr()
-    a.out_dtype = _dev.dtype_code(out_dtype)
-    a.status = st.data_ptr()
-    a.merge = 1 if merge else 0
+    code = _dev.dtype_code
+    a = _lib.AttnArgs(
+        q.data_ptr(), code(q.dtype), B, Hq, Hkv, scale, seq_len.data_ptr(), max_seq_len, v.bits,
+        _lib.KV_PACKED if scores is None else _lib.KV_SCORES, _lib.KVSide() if scores is not None else k.side(),
+        v.side(), None if scores is None else scores.data_ptr(), 0 if scores is None else scores.shape[2],
+        KERNELS[kernel], code(kv_round_dtype), split_tokens, n_splits,
+        None if static_workspace else workspace.data_ptr(), ctx.data_ptr(), out.data_ptr(), code(out_dtype),
+        st.data_ptr(), 1 if merge else 0)
     if trace_scores is not None or trace_v is not None:
         require(kernel == "reference", "Trace outputs come from the exact-order kernel")
         cap = (trace_scores if trace_scores is not None else trace_v).shape[2]

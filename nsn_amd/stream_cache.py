@@ -144,8 +144,13 @@ class StreamingKVCache:
             # each decode step) would leave the GPU idle while the host issues
             # the next launches.  The oldest entries are dropped (a dropped
             # tensor's memory is reused only by later work on the stream).
+            # One length for all -- each decode step of a uniform batch brings a
+            # new one -- is a single fill on the device instead.
             gpu = torch.device(self.device).type == "cuda"
-            t = torch.tensor(key, dtype=torch.int32, pin_memory=gpu).to(self.device, non_blocking=gpu)
+            if min(key) == max(key):
+                t = torch.full((self.batch,), key[0], dtype=torch.int32, device=self.device)
+            else:
+                t = torch.tensor(key, dtype=torch.int32, pin_memory=gpu).to(self.device, non_blocking=gpu)
             if len(self._len_dev) >= 256:
                 self._len_dev.pop(next(iter(self._len_dev)))
             self._len_dev[key] = t
@@ -185,10 +190,12 @@ class StreamingKVCache:
         require(k.shape == v.shape and k.ndim == 4 and tuple(k.shape[:2]) == (self.batch, self.heads)
                 and k.shape[3] == DIM, "Append shape")
         n = k.shape[2]
+        L, C = self.seq_length[slot], self.seq_compressed[slot]
+        # (every sequence alike, a uniform batch's append: checked once, not per sequence)
+        same = counts is None and self.uniform(slot)
         counts = [n] * self.batch if counts is None else [int(c) for c in counts]
         require(len(counts) == self.batch and all(0 <= c <= n for c in counts), "Append counts")
-        L, C = self.seq_length[slot], self.seq_compressed[slot]
-        for b in range(self.batch):
+        for b in range(1 if same else self.batch):
             if L[b] - C[b] + counts[b] > self.tail_cap:
                 raise IntegrityError("Tail overflow: compress before appending more tokens")
             if L[b] + counts[b] > self.block_cap * BLOCK + self.tail_cap:
@@ -203,7 +210,7 @@ class StreamingKVCache:
         kt, vt = self._sides[(slot, "K")].kv.tail, self._sides[(slot, "V")].kv.tail
         lib = _lib.lib()
         dt = _dev.dtype_code(self.dtype)
-        offs = [L[b] - C[b] for b in range(self.batch)]
+        offs = [L[0] - C[0]] if same else [L[b] - C[b] for b in range(self.batch)]
         sdt = _dev.dtype_code(k.dtype)
 
         def launch(kp, vp, ktp, vtp, rows, cnt, off):
@@ -214,7 +221,7 @@ class StreamingKVCache:
             else:
                 rc = lib.nsn_tail_append(kp, vp, rows, cnt, n, ktp, vtp, self.tail_cap, off, dt, _dev.stream())
                 _lib.check(rc, "nsn_tail_append")
-        if len(set(offs)) == 1 and len(set(counts)) == 1:
+        if same or (len(set(offs)) == 1 and len(set(counts)) == 1):
             if counts[0]:
                 launch(k.data_ptr(), v.data_ptr(), kt.data_ptr(), vt.data_ptr(), self.batch * self.heads, counts[0],
                        offs[0])
@@ -313,6 +320,8 @@ class StreamingKVCache:
 
     def post_decode(self):
         for s in range(self.slots):
+            if max(self.seq_length[s]) - min(self.seq_compressed[s]) < 2 * BLOCK:
+                continue   # (no sequence of the slot has a target past its packed prefix)
             self.compress_to(s, [decode_target(L, C) for L, C in zip(self.seq_length[s], self.seq_compressed[s])])
 
     def check_status(self):
