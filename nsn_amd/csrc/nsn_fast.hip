@@ -178,6 +178,8 @@ struct FastParams {
     float *partials;
     int32_t *status;
     int weighted;              // slot weighting: 0 none, 1 two waves per SIMD (5:4), 2 six waves per CU (8:7)
+    int64_t nb_max;            // blocks of max_seq_len
+    int64_t full_waves;        // a small grid: the waves of the full one; 0: the grid is the full one
 };
 
 // Reductions over the 16 lanes of a row with DPP (quad_perm [1,0,3,2],
@@ -969,21 +971,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void at
         // smallest block count per wave with sum_s n_s <= W.  Each wave runs
         // exactly one segment.  Since sum_s ceil(nb_s / P) <= N / P + nstr,
         // the search starts below ceil(N / (W - nstr)).
-        int64_t lo = udivq(N + W - 1, W), hi = wave_max(nb_l);
-        lo = (lo > p.min_blocks) ? lo : p.min_blocks;
-        if (nstr < W) {   // (any P >= ub fits; the answer is the first fit >= lo)
-            int64_t ub = udivq(N + (W - nstr) - 1, W - nstr);
-            ub = (ub > lo) ? ub : lo;
-            hi = (ub < hi) ? ub : hi;
-        }
-        lo = (lo < hi) ? lo : hi;
-        while (lo < hi) {
-            const int32_t mid = static_cast<int32_t>((lo + hi) / 2);
-            const int32_t ns = (nb_l + mid - 1) / mid;
-            if (H * wave_sum(ns < W + 1 ? ns : static_cast<int32_t>(W + 1)) <= W) hi = mid;
-            else lo = mid + 1;
-        }
-        const int32_t P = static_cast<int32_t>(lo);
+        auto blocks_per_wave = [&](const int64_t waves) __attribute__((always_inline)) {
+            int64_t lo = udivq(N + waves - 1, waves), hi = wave_max(nb_l);
+            lo = (lo > p.min_blocks) ? lo : p.min_blocks;
+            if (nstr < waves) {   // (any P >= ub fits; the answer is the first fit >= lo)
+                int64_t ub = udivq(N + (waves - nstr) - 1, waves - nstr);
+                ub = (ub > lo) ? ub : lo;
+                hi = (ub < hi) ? ub : hi;
+            }
+            lo = (lo < hi) ? lo : hi;
+            while (lo < hi) {
+                const int32_t mid = static_cast<int32_t>((lo + hi) / 2);
+                const int32_t ns = (nb_l + mid - 1) / mid;
+                if (H * wave_sum(ns < waves + 1 ? ns : static_cast<int32_t>(waves + 1)) <= waves) hi = mid;
+                else lo = mid + 1;
+            }
+            return static_cast<int32_t>(lo);
+        };
+        const int32_t P = blocks_per_wave(W);
+        // A sequence longer than max_seq_len may need more slots than it has on
+        // the full grid: the small one, whose waves would hold it, refuses it too.
+        int32_t P_full = P;
+        if (p.full_waves && __ballot(nb_l > p.nb_max)) P_full = blocks_per_wave(p.full_waves);
         const int32_t n_l = (nb_l + P - 1) / P;
         const int64_t wincl = H * static_cast<int64_t>(wave_incl_scan32(n_l));   // waves of sequences 0 .. l
         // Wave index w.  The workgroups dispatched first take the first wave
@@ -1030,7 +1039,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void at
         auto blk = [&](int64_t c) { return (c <= nbp) ? c : nbp + (c - nbp + 1) / 3; };
         const int64_t i0 = blk(udivq(cw(k) * U, ctot)), i1 = blk(udivq(cw(k + 1) * U, ctot));
         const int64_t T = at(t_l);
-        if (n <= p.n_splits) {
+        if ((P_full == P ? n : udivq(nb + P_full - 1, P_full)) <= p.n_splits) {
             segment<BITS, QDT, SCORES, GRP, TBF>(p, sh, lane, kvh, i0 * kBlockTok, (i1 * kBlockTok < T) ? i1 * kBlockTok : T,
                                             at(nk_l), at(nv_l), static_cast<int>(k), static_cast<int>(n));
         } else {
@@ -1137,6 +1146,7 @@ int launch_attn_fast(const nsn_attn_args *a, hipStream_t st) {
     // a stream of n blocks touches at most ceil(n / P) + 1 waves
     const int64_t nb_max = (static_cast<int64_t>(a->max_seq_len) + kBlockTok - 1) / kBlockTok;
     p.min_blocks = (nb_max + a->n_splits - 2) / (a->n_splits - 1);
+    p.nb_max = nb_max;
     auto side = [](const nsn_kv_side &s) {
         return FastSide{s.codes, s.mins, s.scales, s.factors, s.blocks, s.block_cap,
                         static_cast<const uint16_t *>(s.tail), s.tail_cap};
@@ -1159,7 +1169,22 @@ int launch_attn_fast(const nsn_attn_args *a, hipStream_t st) {
     // (Measured on C3: 6 per CU 84 us, 4 or 5 per CU 87 us, 8 per CU 100 us.)
     const int per_cu = (a->bits == 3) ? 8 : 6;
     p.weighted = per_cu == 8 ? 1 : (per_cu == 6 ? 2 : 0);
-    const dim3 grid(static_cast<unsigned>(per_cu * (cus[dev] > 0 ? cus[dev] : 256)));
+    const int64_t n_cu = cus[dev] > 0 ? cus[dev] : 256;
+    int64_t waves = per_cu * n_cu;
+    // A call whose waves, min_blocks blocks each, are at most one per SIMD
+    // launches only those: on the full grid half of them sit behind 1024 idle
+    // workgroups, as second-slot waves that wait for a first one's issue slots.
+    // The partition is the full grid's without its weights (min_blocks a wave;
+    // the streams fit, being no more than the waves).
+    // (Split + merge, full grid -> this: 16 kv-heads x 1023 tokens 11.4 -> 10.9 us,
+    // 8 x 8000 16.4 -> 15.2, 5 bits 2 x 4 x 6000 18.6 -> 17.7, 8 x 100 11.7 -> 10.2.)
+    const int64_t small = a->batch * a->heads_kv * ((nb_max + p.min_blocks - 1) / p.min_blocks);
+    if (a->batch <= 64 && small > 0 && small <= 4 * n_cu) {
+        p.full_waves = waves;
+        p.weighted = 0;
+        waves = small;
+    }
+    const dim3 grid(static_cast<unsigned>(waves));
     const bool bf = a->q_dtype == NSN_DTYPE_BF16;
 #define NSN_FAST_LAUNCH2(B_, Q_, S_, G_, T_) \
     hipLaunchKernelGGL((attn_fast_kernel<B_, Q_, S_, G_, T_>), grid, dim3(64), 0, st, p)

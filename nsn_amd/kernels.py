@@ -113,10 +113,12 @@ def decode_split(batch, heads_kv, max_len, kernel):
     workgroups of the exact-order kernel, of which 3 fit on a CU), in up to
     128 splits (more make the merge longer than they save).  Measured, 256
     tokens a split against this rule: fast 1 x 16 kv-heads x 1023 tokens 20.0
-    -> 11.4 us, 5 x 4 x 6500 24.0 -> 18.3, 64 x 8 x 500 29.5 -> 18.4, 1 x 8 x
-    32000 23.7 -> 22.6 (64 tokens: 24.4); exact-order 1 x 16 x 1023 45 ->
-    15.5, 1 x 8 x 4133 45 -> 24.0, 4 x 8 x 2000 31.2 -> 24.6.  The fast kernel takes one slot more than there are splits: its
-    blocks per wave are bounded by blocks / (slots - 1).
+    -> 10.9 us, 5 x 4 x 6500 24.0 -> 18.3, 64 x 8 x 500 29.5 -> 18.4, 1 x 8 x
+    32000 23.7 -> 20.9 (64 tokens: 24.4); exact-order 4 x 8 x 2000 31.2 (128
+    tokens) -> 24.6, and with a slower restore than today's 1 x 16 x 1023 49.5
+    -> 17.5, 1 x 8 x 4133 55.7 -> 30.6.  The fast kernel takes one slot more
+    than there are splits: its blocks per wave are bounded by blocks /
+    (slots - 1).
     """
     split, n = default_split(batch, heads_kv, max_len)
     fine = max(1, min(128, (2048 if kernel == "fast" else 1024) // max(1, batch * heads_kv)))

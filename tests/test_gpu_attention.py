@@ -610,3 +610,37 @@ def test_vf01_normal_fixtures_on_the_fast_kernel(arm):
         ref = _fixture_oracle(a, f, "float32" if arm == "V_FUSED" else "bfloat16")
         ok, err = within(ctx.cpu().numpy().reshape(2, 128), ref)
         assert ok, (f["id"], err)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,lengths,split", [
+    (2, 8, 2, [63, 1], None),             # one wave a stream, tails only
+    (3, 16, 4, [1500, 64, 700], None),    # one block a wave, streams of different lengths
+    (2, 32, 16, [2048, 1999], None),      # 1024 waves: the largest small grid of 256 CUs
+    (2, 32, 16, [2049, 65], None),        # 1056: the full grid
+    (1, 8, 2, [1300], 512),               # several blocks a wave
+    (64, 4, 1, [(37 * i) % 200 + 1 for i in range(64)], None),
+])
+def test_fast_small_grids_vs_oracle(B, Hq, Hkv, lengths, split):
+    """A call that needs at most one wave per SIMD launches only those waves."""
+    k, v, qb, kk, vv, seq = make_case(41, B, Hq, Hkv, lengths)
+    _, ctx = kernels.decode_attention(qb.to(DEV), kk, vv, seq, kernel="fast", split_tokens=split,
+                                      kv_round_dtype=torch.float16)
+    ok, err = within(ctx.cpu().numpy(), oracle_ctx(k, v, qb, lengths, 3, "float32"))
+    assert ok, err
+
+
+@pytest.mark.parametrize("length,refused", [(64, False), (128, False), (130, True), (1000, True)])
+def test_fast_small_grid_refuses_what_the_slots_cannot_hold(length, refused):
+    """Device lengths past max_seq_len: a sequence of more one-block waves than
+    its two slots raises NSN_ST_WORKSPACE, though a small grid's waves would
+    hold it; one that fits its slots matches the oracle."""
+    from nsn_amd import _dev, _lib
+    k, v, qb, kk, vv, seq = make_case(42, 1, 8, 2, [length])
+    ws = torch.zeros(kernels.workspace_floats(1, 8, 2), dtype=torch.float32, device=DEV)
+    st = _dev.new_status(DEV)
+    _, ctx = kernels.decode_attention(qb.to(DEV), kk, vv, seq, max_seq_len=64, kernel="fast", check=False,
+                                      status=st, workspace=ws)
+    assert bool(_dev.read_status(st) & _lib.ST_WORKSPACE) == refused
+    if not refused:
+        ok, err = within(ctx.cpu().numpy(), oracle_ctx(k, v, qb, [length], 3, "float32"))
+        assert ok, err
