@@ -374,11 +374,12 @@ class PackedKVCache(Cache):
         return out
 
     def _workspace(self, L):
-        _, n = kernels.decode_split(self.batch, self.heads, L, "fast")
+        # one size for every length: a captured step keeps the buffer's address
+        # while eager steps at other lengths run
+        n = kernels.decode_slots(self.batch, self.heads, max(L, self.cap_len), "fast")
         need = kernels.workspace_floats(self.batch, self.heads_q, n)
         if self._ws is None or self._ws.numel() < need:
-            self._ws = torch.empty(max(need, 2 * (0 if self._ws is None else self._ws.numel())),
-                                   dtype=torch.float32, device=self.store.device)
+            self._ws = torch.empty(need, dtype=torch.float32, device=self.store.device)
         return self._ws
 
 

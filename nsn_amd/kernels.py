@@ -128,6 +128,15 @@ def decode_split(batch, heads_kv, max_len, kernel):
     return split, max(2, n) if kernel == "fast" else n
 
 
+def decode_slots(batch, heads_kv, max_len, kernel):
+    """The most splits decode_split gives any context of up to max_len tokens
+    (its count is not monotonic: 16 kv-heads take 129 at 8192 tokens, 66 at
+    8256), for a workspace that must not move when the length changes."""
+    want = math.ceil(4096 / max(1, batch * heads_kv))
+    fine = max(1, min(128, (2048 if kernel == "fast" else 1024) // max(1, batch * heads_kv)))
+    return max(2, min(want, math.ceil(max_len / 256)), min(fine, math.ceil(max_len / BLOCK)) + 1)
+
+
 def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=None, scores=None,
                      kernel="reference", kv_round_dtype=None, split_tokens=None, out_dtype=torch.bfloat16,
                      scale=SCALE, status=None, check=True, workspace=None, out=None, ctx=None, merge=True,

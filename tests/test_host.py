@@ -135,6 +135,24 @@ def test_decode_split_covers_context_and_bounds_its_slots():
                 assert -(-blocks // (n - 1)) <= split // 64     # blocks of a wave: what the split asks for
 
 
+@pytest.mark.parametrize("B,Hq,H", [(1, 16, 16), (1, 32, 8), (3, 28, 4), (64, 8, 8), (1, 1, 1)])
+def test_decode_workspace_does_not_move_with_the_length(B, Hq, H):
+    """The adapter's decode workspace, whose address a captured step holds:
+    one buffer for every length up to the capacity, in any order of lengths."""
+    from types import SimpleNamespace
+
+    from nsn_amd.adapter import PackedKVCache
+    cap = 9000
+    cache = SimpleNamespace(batch=B, heads=H, heads_q=Hq, cap_len=cap, _ws=None, store=SimpleNamespace(device="cpu"))
+    ws = PackedKVCache._workspace(cache, cap)
+    for L in range(1, cap + 1):
+        n = kernels.decode_split(B, H, L, "fast")[1]
+        assert n <= kernels.decode_slots(B, H, cap, "fast")
+        assert kernels.decode_split(B, H, L, "reference")[1] <= kernels.decode_slots(B, H, cap, "reference")
+        if n > kernels.decode_split(B, H, cap, "fast")[1] or L % 500 == 0:
+            assert PackedKVCache._workspace(cache, L) is ws and ws.numel() >= kernels.workspace_floats(B, Hq, n)
+
+
 def _cpu_fixture(kind):
     """The reference's negative fixtures that fail structural checks (loop_kv_vf01_contract.py:98-120)."""
     a = gi.vf01_fixture(64, 65, "mixed_codes")
