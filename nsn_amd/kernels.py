@@ -172,8 +172,10 @@ def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=
         max_seq_len = int(seq_len.max().item())
     if split_tokens is None:
         split_tokens, n_splits = decode_split(B, Hkv, max_seq_len, kernel)
-        if static_workspace and workspace_floats(B, Hq, n_splits) > _lib.STATIC_SCRATCH_FLOATS:
-            split_tokens, n_splits = default_split(B, Hkv, max_seq_len)   # (fewer slots: what the scratch holds)
+        room = _lib.STATIC_SCRATCH_FLOATS if static_workspace else None if workspace is None else workspace.numel()
+        if room is not None and workspace_floats(B, Hq, n_splits) > room:
+            # fewer slots, for a workspace sized by default_split (which merge=False callers read)
+            split_tokens, n_splits = default_split(B, Hkv, max_seq_len)
     else:
         n_splits = max(1, math.ceil(max_seq_len / split_tokens))
     if kernel == "fast":

@@ -557,6 +557,23 @@ def test_empty_and_over_capacity_sequences_with_device_lengths(kernel):
     assert ok, err
 
 
+@pytest.mark.parametrize("kernel", ["fast", "reference"])
+def test_workspace_sized_by_default_split_is_used(kernel):
+    """A call that names no split keeps a caller's workspace that holds
+    default_split's partials but not the finer split's: it is written, and the
+    result is the named split's bit for bit."""
+    k, v, qb, kk, vv, seq = make_case(11, 1, 8, 2, [1000])
+    split, n = kernels.default_split(1, 2, 1000)
+    n = max(2, n) if kernel == "fast" else n
+    need = kernels.workspace_floats(1, 8, n)
+    assert kernels.workspace_floats(1, 8, kernels.decode_split(1, 2, 1000, kernel)[1]) > need
+    ws = torch.full((need,), float("nan"), dtype=torch.float32, device=DEV)
+    got = kernels.decode_attention(qb.to(DEV), kk, vv, seq, max_seq_len=1000, kernel=kernel, workspace=ws)
+    assert not bool(torch.isnan(ws).all())
+    want = kernels.decode_attention(qb.to(DEV), kk, vv, seq, max_seq_len=1000, kernel=kernel, split_tokens=split)
+    assert torch.equal(got[1], want[1]) and torch.equal(got[0], want[0])
+
+
 @pytest.mark.parametrize("Hq,Hkv,bits", [(8, 2, 3), (32, 4, 3), (8, 2, 5), (16, 8, 5), (16, 2, 5)])
 def test_fast_bf16_tails_vs_oracle(Hq, Hkv, bits):
     """bf16 tails (the reference's dtype, loop_kv_qk01_kernel.py:66-69) on the
