@@ -236,10 +236,11 @@ struct Parts {
 #pragma clang diagnostic ignored "-Winline-asm"
 // 16 bytes per lane from global memory straight into LDS at M0 + 16*lane,
 // with the non-temporal hint: a workgroup streams each block of its context
-// once (C4 last chunk 1241-1242 -> 1222-1228 us).
+// once (C4 last chunk 1241-1242 -> 1222-1228 us).  The s_nop is the wait state
+// that a load to LDS needs after a scalar write of M0.
 __device__ __forceinline__ void dma16(const void *src, void *dst) {
     const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst));
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(src), "s"(lds) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(src), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 

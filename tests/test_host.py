@@ -59,6 +59,21 @@ def test_library_rejects_bad_arguments_without_gpu_work():
     assert lib.nsn_prefill_attention(pa, None) == _lib.NSN_EINVAL    # the V tail is missing
 
 
+def test_lds_loads_wait_for_their_m0_write():
+    """A load to LDS needs one wait state after a scalar write of M0 (its LDS
+    address): without it the load may go to the previous address.  The compiler
+    inserts it around its own builtins but not inside an asm block."""
+    strings = []
+    for src in sorted((ROOT / "nsn_amd" / "csrc").glob("*.h*")):
+        for text in re.findall(r'asm volatile\(((?:\s*"(?:[^"\\]|\\.)*")+)', src.read_text()):
+            lines = [ln.strip() for ln in "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', text)).split("\\n\\t")]
+            for a, b in zip(lines, lines[1:]):
+                if re.match(r"s_\w+ m0\b", a):
+                    strings.append((src.name, lines))
+                    assert b.startswith("s_nop"), (src.name, lines)
+    assert len(strings) == 3, strings
+
+
 def test_device_position_appends_reject_bad_arguments_without_gpu_work():
     """nsn_tail_append_to, nsn_tail_append_cast and nsn_rope_append validate on the host before any
     launch (fake, never dereferenced addresses stand in for device buffers)."""
