@@ -219,7 +219,10 @@ struct PrefillParams {
 // at once, and a tile with one split left writes its output itself.
 // Workspace: per (tile, split) 256 pairs (running maximum, weight sum), then
 // per (tile, split) the unnormalised O^T in register order, [8 waves][16][64
-// lanes] float4.  A weight sum of kDone marks a tile without partials.
+// lanes] float4.  A weight sum of kDone marks a slot without partials: every
+// slot of a tile whose output is written, and the splits that left at once.
+// (The maximum cannot mark them: it is also -inf where all of a split's scores
+// are NaN, or its tokens masked, and its NaN must reach the output.)
 constexpr int kMaxSplits = 16, kSplitBlocks = 8;
 constexpr float kDone = -1.f;
 struct Parts {
@@ -536,7 +539,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     int splits = nblk / kSplitBlocks;
     splits = splits < 1 ? 1 : (splits < p.splits ? splits : p.splits);
     if (split >= splits) {
-        if (tid < kQTile) parts().ml[tid] = float2{-INFINITY, 0.f};
+        if (tid < kQTile) parts().ml[tid] = float2{-INFINITY, kDone};
         return;
     }
     const int j0 = static_cast<int>(static_cast<int64_t>(nblk) * split / splits);
@@ -848,7 +851,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
 #pragma unroll
     for (int s = 0; s < kMaxSplits; ++s) {
         m[s] = -INFINITY;
-        w[s] = 0.f;
+        w[s] = kDone;
         if (s < p.splits) {
             const float2 v = Parts(p.part, tiles, p.splits, tile, s).ml[32 * wave + (l & 31)];
             m[s] = v.x;
@@ -861,8 +864,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillParams p) {
     float o[4][4] = {};
 #pragma unroll
     for (int s = 0; s < kMaxSplits; ++s) {
-        if (s < p.splits && m[s] != -INFINITY) {   // (a split that saw no token of the row has no weight)
-            const float a = __builtin_amdgcn_exp2f(m[s] - M);
+        if (w[s] != kDone) {   // (true for NaN)
+            const float a = (m[s] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[s] - M);   // (0 * NaN stays NaN)
             L = __builtin_fmaf(a, w[s], L);
             const float4 *src = Parts(p.part, tiles, p.splits, tile, s).acc + (wave * 16 + 4 * ct) * 64 + l;
 #pragma unroll

@@ -206,6 +206,47 @@ def test_prefill_context_splits_append(monkeypatch):
     assert bool((d <= 2.0 ** -10 * got[0][0].float().abs() + 2.0 ** -10).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("where,Hq,n,L,splits", [
+    ("k_factors", 2, 90, 1920, 4),   # every block of the second of four splits: NaN scores only
+    ("k_chunk", 1, 512, 512, 2),     # a NaN key in each chunk block; the later tile's second split is the chunk
+    ("v_chunk", 3, 600, 384, 2),     # a NaN value in a split where the earlier queries of a head see no token
+    ("v_factors", 2, 90, 1920, 4),
+])
+def test_prefill_context_splits_keep_nonfinite_values(monkeypatch, where, Hq, n, L, splits, dtype):
+    """Nonfinite K/V in one split only: the NaN outputs and the status are those
+    of the unsplit call, the other rows within one rounding of the output and
+    one of the weights (whose scale moves with the split's maximum)."""
+    from nsn_amd import _dev, _lib
+    rng = np.random.default_rng(45)
+    (kk, seq), (vv, _) = (cache.pack_sequences(torch.from_numpy(normal_tokens(rng, (1, 1), L)).to(DEV), [L],
+                                               tail_dtype=dtype) for _ in range(2))
+    q, kc, vc = (torch.from_numpy(normal_tokens(rng, (1, h), n)).to(DEV, dtype) for h in (Hq, 1, 1))
+    if where == "k_factors":
+        kk.factor.view(1, 1, -1, 64)[:, :, 8:16] = float("nan")
+    elif where == "v_factors":
+        vv.factor.view(1, 1, -1, 64)[:, :, 8:16] = float("nan")
+    elif where == "k_chunk":
+        kc[:, :, ::64] = float("nan")
+    else:
+        vc[:, :, -1] = float("nan")
+    got = []
+    for s in (1, splits):
+        monkeypatch.setattr(kernels._lib.lib(), "nsn_prefill_splits", lambda *a, s=s: s)
+        st = _dev.new_status(DEV)
+        out = kernels.prefill_attention(q, kk, vv, seq, kc, vc, check=False, status=st, precise_weights=False)
+        got.append((out.float(), _dev.read_status(st)))
+    (one, s1), (many, s2) = got
+    print(f"nonfinite {where}: {int(one.isnan().sum())} NaN of {one.numel()} unsplit, {int(many.isnan().sum())} split",
+          flush=True)
+    assert s1 == s2 == _lib.ST_NONFINITE_OUTPUT
+    assert bool(one.isnan().any()) and torch.equal(one.isnan(), many.isnan())
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    d = (one - many).abs().nan_to_num(0.0)
+    # N(0,1) values: a row's weights, rounded twice, move it by at most 2u of the attended |v| (< 4)
+    assert bool((d <= 2 * u * one.abs().nan_to_num(0.0) + 8 * u).all())
+
+
 def test_prefill_repeats_bit_for_bit():
     """Every read of a product's result waits for it: the same call twice gives
     the same bits (a maximum read too early moves only the last place)."""
