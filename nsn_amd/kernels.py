@@ -173,8 +173,9 @@ def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=
     if split_tokens is None:
         split_tokens, n_splits = decode_split(B, Hkv, max_seq_len, kernel)
         room = _lib.STATIC_SCRATCH_FLOATS if static_workspace else None if workspace is None else workspace.numel()
-        if room is not None and workspace_floats(B, Hq, n_splits) > room:
-            # fewer slots, for a workspace sized by default_split (which merge=False callers read)
+        if not merge or (room is not None and workspace_floats(B, Hq, n_splits) > room):
+            # the partials of a call without its merge are read at default_split's
+            # stride; a workspace of default_split's size has no room for more slots
             split_tokens, n_splits = default_split(B, Hkv, max_seq_len)
     else:
         n_splits = max(1, math.ceil(max_seq_len / split_tokens))
@@ -239,6 +240,8 @@ def decode_attention(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_
     cap >= max_seq_len; reference kernel only) receive what the kernel itself
     computed for every token t < seq_len[b]: its scores and the V rows it
     multiplied (the TRACE stores of loop_kv_vf01_kernel.py:104,113).
+    ``merge=False`` leaves the partials in ``workspace``, in default_split's
+    count where ``split_tokens`` names none.
     ``validate_lengths`` (default: with ``check`` or without ``max_seq_len``)
     copies the lengths and block counts to the host and checks them against
     the buffers; callers that built them from tensor shapes pass False.

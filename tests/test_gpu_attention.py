@@ -574,6 +574,28 @@ def test_workspace_sized_by_default_split_is_used(kernel):
     assert torch.equal(got[1], want[1]) and torch.equal(got[0], want[0])
 
 
+@pytest.mark.parametrize("kernel", ["fast", "reference"])
+def test_partials_without_merge_have_default_splits_layout(kernel):
+    """merge=False without a named split, in a workspace with room for finer
+    ones: the partials lie at default_split's stride, for the caller's merge."""
+    from nsn_amd import _dev, _lib
+    k, v, qb, kk, vv, seq = make_case(12, 1, 8, 2, [1000])
+    split, n = kernels.default_split(1, 2, 1000)
+    n = max(2, n) if kernel == "fast" else n
+    assert kernels.decode_split(1, 2, 1000, kernel)[1] > n
+    ws = torch.zeros(kernels.workspace_floats(1, 8, 200), dtype=torch.float32, device=DEV)
+    st = _dev.new_status(DEV)
+    kernels.decode_attention(qb.to(DEV), kk, vv, seq, max_seq_len=1000, kernel=kernel, workspace=ws, merge=False,
+                             status=st)
+    ctx = torch.zeros((1, 8, 128), dtype=torch.float32, device=DEV)
+    out = torch.zeros((1, 8, 128), dtype=torch.bfloat16, device=DEV)
+    rc = _lib.lib().nsn_attention_merge(ws.data_ptr(), 1, 8, n, ctx.data_ptr(), out.data_ptr(), _lib.DTYPE_BF16,
+                                        st.data_ptr(), _dev.stream())
+    assert rc == _lib.NSN_OK and _dev.read_status(st) == 0
+    want = kernels.decode_attention(qb.to(DEV), kk, vv, seq, max_seq_len=1000, kernel=kernel, split_tokens=split)
+    assert torch.equal(ctx, want[1]) and torch.equal(out, want[0])
+
+
 @pytest.mark.parametrize("Hq,Hkv,bits", [(8, 2, 3), (32, 4, 3), (8, 2, 5), (16, 8, 5), (16, 2, 5)])
 def test_fast_bf16_tails_vs_oracle(Hq, Hkv, bits):
     """bf16 tails (the reference's dtype, loop_kv_qk01_kernel.py:66-69) on the
