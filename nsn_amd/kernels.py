@@ -98,43 +98,73 @@ def workspace_floats(batch, heads_q, n_splits):
 
 def default_split(batch, heads_kv, max_len, target_units=4096, min_split=256):
     """Split the context so that batch*heads_kv*splits covers the 256 CUs several times."""
-    want = max(1, math.ceil(target_units / max(1, batch * heads_kv)))
-    split = max(min_split, math.ceil(max_len / want / BLOCK) * BLOCK)
-    split = min(split, math.ceil(max_len / BLOCK) * BLOCK)
-    return max(BLOCK, split), max(1, math.ceil(max_len / max(BLOCK, split)))
+    want = -(-target_units // (batch * heads_kv or 1))
+    split = -(-max_len // (want * BLOCK)) * BLOCK
+    if split < min_split:
+        split = min(min_split, -(-max_len // BLOCK) * BLOCK or BLOCK)
+    return split, -(-max_len // split) or 1
 
 
-def decode_split(batch, heads_kv, max_len, kernel):
+def _finest_split(batch, heads_kv, group, blocks, coarse, kernel):
+    """The most splits of `blocks` blocks that pay (`coarse`: default_split's
+    partials).  Measured per shape with every blocks-per-wave count:
+
+    - exact-order: the 768 workgroups that run at once (3 per CU); a second
+      round costs more than it saves (128 blocks, 20 kv-heads of 7 queries:
+      32 splits 78.6 us, 43 92.9; 512 kv-heads x 3 blocks: 1 32.3, 2 45.6);
+    - fast: 1024 waves, the small grid, in at most the 64 partials that the
+      merge holds in registers (8 kv-heads x 79 blocks: 40 partials 12.6 us,
+      79 14.5; 16 x 256: 64 18.0, 128 18.9; one block each at 1 x 16 x 1023);
+    - fast, where a wave of that would walk four blocks or more: 2048 waves, if
+      their partials stay within 4.3 MB (about an XCD's L2; 512 kv-heads of 4
+      queries x 8 blocks: 2 splits 22.1 us, 4 19.3; 256 of 7 x 16 blocks,
+      7.6 MB: 4 26.7, 8 31.0), and past 64 partials for up to 8 kv-heads, whose
+      128 still are the small grid (8 x 300: 60 19.4, 100 18.3), or where
+      default_split passes them already (16 x 375: 75 23.8, 125 22.2).
+    """
+    streams = batch * heads_kv or 1
+    if kernel != "fast":
+        return min(128, 768 // streams) or 1
+    fine = min(64, 1024 // streams) or 1
+    if blocks > 3 * fine:
+        wide = min(128 if streams <= 8 or coarse > 64 else 64, 2048 // streams) or 1
+        if streams * group * wide <= 8192:
+            return wide
+    return fine
+
+
+def decode_split(batch, heads_kv, max_len, kernel, group=1):
     """(split_tokens, n_splits) of a decode call that names none: default_split,
-    cut finer while the call is too small to fill the GPU with it.
-
-    A short context is bound by the blocks one wave walks in series, so it is
-    spread over up to 2048 waves (the fast kernel's resident ones; 1024
-    workgroups of the exact-order kernel, of which 3 fit on a CU), in up to
-    128 splits (more make the merge longer than they save).  Measured, 256
-    tokens a split against this rule: fast 1 x 16 kv-heads x 1023 tokens 20.0
-    -> 10.9 us, 5 x 4 x 6500 24.0 -> 18.3, 64 x 8 x 500 29.5 -> 18.4, 1 x 8 x
-    32000 23.7 -> 20.9 (64 tokens: 24.4); exact-order 4 x 8 x 2000 31.2 (128
-    tokens) -> 24.6, and with a slower restore than today's 1 x 16 x 1023 49.5
-    -> 17.5, 1 x 8 x 4133 55.7 -> 30.6.  The fast kernel takes one slot more
-    than there are splits: its blocks per wave are bounded by blocks /
-    (slots - 1).
+    cut finer (_finest_split) where that leaves a wave fewer blocks to walk in
+    series, which is what bounds a short context.  The fast kernel takes one
+    slot more than there are splits: its blocks per wave are bounded by blocks /
+    (slots - 1).  Kernel times, default_split -> this: fast 1 x 16 kv-heads x
+    1023 tokens 15.7 -> 11.3 us, 5 x 4 x 6500 (7 queries each) 20.0 -> 18.3,
+    64 x 8 x 500 22.3 -> 17.6; exact-order 4 x 8 x 2000 48.1 -> 31.3, 1 x 8 x
+    4133 48.2 -> 21.2.
     """
     split, n = default_split(batch, heads_kv, max_len)
-    fine = max(1, min(128, (2048 if kernel == "fast" else 1024) // max(1, batch * heads_kv)))
-    finer = max(BLOCK, math.ceil(max_len / fine / BLOCK) * BLOCK)
-    if finer < split:
-        split, n = finer, math.ceil(max_len / finer) + (1 if kernel == "fast" else 0)
-    return split, max(2, n) if kernel == "fast" else n
+    blocks = -(-max_len // BLOCK) or 1
+    if kernel == "fast":
+        spare = 1
+        walk = -(-blocks // (n - 1)) if n > 2 else blocks
+        if n < 2:
+            n = 2
+    else:
+        spare, walk = 0, split // BLOCK
+    take = -(-blocks // _finest_split(batch, heads_kv, group, blocks, -(-blocks // walk), kernel))
+    if take < walk and take * BLOCK <= split:
+        return take * BLOCK, -(-blocks // take) + spare
+    return split, n
 
 
 def decode_slots(batch, heads_kv, max_len, kernel):
     """The most splits decode_split gives any context of up to max_len tokens
-    (its count is not monotonic: 16 kv-heads take 129 at 8192 tokens, 66 at
-    8256), for a workspace that must not move when the length changes."""
-    want = math.ceil(4096 / max(1, batch * heads_kv))
-    fine = max(1, min(128, (2048 if kernel == "fast" else 1024) // max(1, batch * heads_kv)))
-    return max(2, min(want, math.ceil(max_len / 256)), min(fine, math.ceil(max_len / BLOCK)) + 1)
+    and any group (its count is not monotonic in the length), for a workspace
+    that must not move when the length changes."""
+    streams = max(1, batch * heads_kv)
+    fine = max(1, min(128, (2048 if kernel == "fast" else 768) // streams))
+    return max(2, min(math.ceil(4096 / streams), math.ceil(max_len / 256)), min(fine, math.ceil(max_len / BLOCK)) + 1)
 
 
 def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=None, scores=None,
@@ -171,7 +201,7 @@ def _decode_args(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_len=
     if max_seq_len is None:
         max_seq_len = int(seq_len.max().item())
     if split_tokens is None:
-        split_tokens, n_splits = decode_split(B, Hkv, max_seq_len, kernel)
+        split_tokens, n_splits = decode_split(B, Hkv, max_seq_len, kernel, Hq // Hkv)
         room = _lib.STATIC_SCRATCH_FLOATS if static_workspace else None if workspace is None else workspace.numel()
         if not merge or (room is not None and workspace_floats(B, Hq, n_splits) > room):
             # the partials of a call without its merge are read at default_split's

@@ -150,6 +150,33 @@ def test_decode_split_covers_context_and_bounds_its_slots():
                 assert -(-blocks // (n - 1)) <= split // 64     # blocks of a wave: what the split asks for
 
 
+def test_decode_split_stays_within_what_runs_and_merges_well():
+    """Finer splits than default_split's: the exact-order kernel's workgroups
+    run at once (768); the fast kernel's waves are the small grid's 1024 in at
+    most 64 partials, or 2048 with at most 4.3 MB of partials, past 64 of them
+    only for up to 8 kv-heads or where default_split already passes them."""
+    finer = 0
+    for S in (1, 4, 8, 12, 16, 20, 24, 32, 48, 64, 128, 256, 512, 1024, 3000):
+        for group in (1, 4, 5, 7, 16):
+            for blocks in list(range(1, 130)) + [188, 256, 257, 320, 321, 375, 400, 500, 512, 1000]:
+                L = 64 * blocks - 17
+                base, nb = kernels.default_split(1, S, L)
+                for kernel in ("fast", "reference"):
+                    split, n = kernels.decode_split(1, S, L, kernel, group)
+                    assert split % 64 == 0 and split * n >= L and n <= kernels.decode_slots(1, S, L, kernel)
+                    if (split, n) == (base, max(2, nb) if kernel == "fast" else nb):
+                        continue
+                    finer += 1
+                    assert split <= base
+                    if kernel == "reference":
+                        assert S * n <= 768 and n >= nb
+                        continue
+                    waves, coarse = n - 1, -(-blocks // -(-blocks // (max(2, nb) - 1)))
+                    assert waves >= coarse and waves <= (128 if coarse > 64 or S <= 8 else 64)
+                    assert S * waves <= (2048 if S * group * waves <= 8192 else 1024)
+    assert finer > 1000
+
+
 @pytest.mark.parametrize("B,Hq,H", [(1, 16, 16), (1, 32, 8), (3, 28, 4), (64, 8, 8), (1, 1, 1)])
 def test_decode_workspace_does_not_move_with_the_length(B, Hq, H):
     """The adapter's decode workspace, whose address a captured step holds:
