@@ -328,7 +328,7 @@ def prepare_decode(q, k: Optional[PackedKV], v: PackedKV, seq_len, *, max_seq_le
 
 
 def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, k_chunk, v_chunk, *, scale=SCALE,
-                      status=None, check=True, out=None, append=False, precise_weights=None):
+                      status=None, check=True, out=None, append=False, precise_weights=None, max_ctx_len=None):
     """Chunked-prefill attention over a packed context (C4's prefill step).
 
     q [B, Hq, n, 128]; k_chunk, v_chunk [B, Hkv, n, 128] (the chunk's own K/V;
@@ -347,6 +347,13 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
     as bf16 hi + lo (~2^-17 relative) instead of one bf16 rounding, at ~24 %
     more kernel time; None = only when there is no context (k is None), where
     the first queries attend a handful of tokens.
+
+    Where the call has few tiles for its context, the context is split and the
+    splits merged by a second kernel, through a workspace of 130 KB per tile
+    and split (up to 67 MB for chunks of 512) allocated for the call.  ``max_ctx_len``: the
+    longest context, where the host knows it; it only chooses the split count
+    (without it, and without ``check``, the cache's capacity stands for it, and
+    a short context on a large cache pays 3-7 us for a merge of nothing).
     """
     _dev.require_gpu(q, k_chunk, v_chunk, ctx_len)
     qshape, cshape, qdt = q.shape, k_chunk.shape, q.dtype
@@ -374,6 +381,7 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
         bits = k.bits
         if check:
             L = ctx_len.cpu().numpy().astype(np.int64)
+            max_ctx_len = int(L.max(initial=0))
             nk = k.blocks.cpu().numpy().astype(np.int64) if k.codes is not None else np.zeros_like(L)
             nv = v.blocks.cpu().numpy().astype(np.int64) if v.codes is not None else np.zeros_like(L)
             require(np.array_equal(nk, nv), "K/V packed block counts differ")
@@ -410,10 +418,14 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
     a.append = 1 if append else 0
     a.precise_weights = 1 if (k is None if precise_weights is None else precise_weights) else 0
     # few tiles (one long sequence, a short chunk): split the context too.  The
-    # lengths stay on the device, so the capacity bounds them here; the kernel
-    # uses no more splits than the actual length pays for.
-    lib = _lib.lib()
-    splits, ws = lib.nsn_prefill_splits(B, Hq, Hkv, n, a.k.block_cap + (a.k.tail_cap + n) // BLOCK + 2), None
+    # capacity bounds lengths that stay on the device; of known ones the kernel
+    # uses a split per 8 blocks at most, and no other is launched (128 queries x
+    # 32 heads on a 32K cache: over 256 tokens 29.6 -> 23.5 us, over 1024 36.1
+    # -> 32.5).
+    lib, ws = _lib.lib(), None
+    splits = lib.nsn_prefill_splits(B, Hq, Hkv, n, a.k.block_cap + (a.k.tail_cap + n) // BLOCK + 2)
+    if splits > 1 and max_ctx_len is not None:
+        splits = max(1, min(splits, (-(-max_ctx_len // BLOCK) - (-n // BLOCK)) // 8))
     if splits > 1:
         ws = torch.empty(lib.nsn_prefill_workspace_floats(B, Hq, Hkv, n, splits), dtype=torch.float32, device=q.device)
     rc = lib.nsn_prefill_attention_split(a, splits, ws if ws is None else ws.data_ptr(), _dev.stream())

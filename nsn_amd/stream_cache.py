@@ -349,6 +349,7 @@ class StreamingKVCache:
         sequence of the slot has less than one block of context: its first
         queries attend a handful of tokens."""
         kw.setdefault("precise_weights", min(self.seq_length[slot]) < BLOCK)
+        kw.setdefault("max_ctx_len", max(self.seq_length[slot]))
         if append:
             n = k_chunk.shape[2]
             L, C = self.seq_length[slot], self.seq_compressed[slot]

@@ -336,3 +336,24 @@ def test_prefill_append_without_room():
     for a, b in zip(before, _state(c)):
         assert torch.equal(a, b)
     assert c.seq_length[0] == [150]
+
+
+def test_prefill_splits_follow_the_length_not_the_capacity(monkeypatch):
+    """The chunks of one sequence on a large cache: as many splits as the blocks
+    it holds fill (8 each), none while they fill only one, alike where the call
+    reads the lengths back."""
+    from nsn_amd import kernels
+    lib, used = kernels._lib.lib(), []
+    real = lib.nsn_prefill_attention_split
+
+    def launch(a, splits, ws, stream):
+        used.append(splits)
+        return real(a, splits, ws, stream)
+    monkeypatch.setattr(lib, "nsn_prefill_attention_split", launch)
+    c = StreamingKVCache(1, 1, 8, 32768, max_append=512, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    for i in range(13):
+        q, k, v = (torch.randn((1, h, 128, 128), generator=g, device=DEV).half() for h in (32, 8, 8))
+        c.prefill(0, q, k, v, append=True, check=i % 2 == 1)
+        c.post_prefill()
+    assert used == [max(1, (2 * i + 2) // 8) for i in range(13)]
