@@ -350,10 +350,11 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
 
     Where the call has few tiles for its context, the context is split and the
     splits merged by a second kernel, through a workspace of 130 KB per tile
-    and split (up to 67 MB for chunks of 512) allocated for the call.  ``max_ctx_len``: the
-    longest context, where the host knows it; it only chooses the split count
-    (without it, and without ``check``, the cache's capacity stands for it, and
-    a short context on a large cache pays 3-7 us for a merge of nothing).
+    and split (up to 67 MB for chunks of 512) allocated for the call.
+    ``max_ctx_len``: the longest context, where the host knows it; it only
+    chooses the split count (without it, and without ``check``, the cache's
+    capacity stands for it, and a short context on a large cache pays 3-7 us
+    for a merge of nothing).
     """
     _dev.require_gpu(q, k_chunk, v_chunk, ctx_len)
     qshape, cshape, qdt = q.shape, k_chunk.shape, q.dtype
@@ -418,14 +419,18 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
     a.append = 1 if append else 0
     a.precise_weights = 1 if (k is None if precise_weights is None else precise_weights) else 0
     # few tiles (one long sequence, a short chunk): split the context too.  The
-    # capacity bounds lengths that stay on the device; of known ones the kernel
-    # uses a split per 8 blocks at most, and no other is launched (128 queries x
-    # 32 heads on a 32K cache: over 256 tokens 29.6 -> 23.5 us, over 1024 36.1
-    # -> 32.5).
+    # capacity bounds lengths that stay on the device.  The kernel uses a split
+    # per 8 blocks at most: no other is launched for the blocks that the longest
+    # sequence holds, or, of unknown lengths, for the packed capacity and what
+    # the streaming policy leaves in a tail (128 queries x 32 heads on a 32K
+    # cache: over 256 tokens 29.6 -> 23.5 us, over 1024 36.1 -> 32.5).
     lib, ws = _lib.lib(), None
     splits = lib.nsn_prefill_splits(B, Hq, Hkv, n, a.k.block_cap + (a.k.tail_cap + n) // BLOCK + 2)
-    if splits > 1 and max_ctx_len is not None:
-        splits = max(1, min(splits, (-(-max_ctx_len // BLOCK) - (-n // BLOCK)) // 8))
+    if splits > 1:
+        tail = a.k.tail_cap // BLOCK
+        held = (-(-max_ctx_len // BLOCK) if max_ctx_len is not None
+                else a.k.block_cap + min(tail, 2) if a.k.block_cap else tail)
+        splits = max(1, min(splits, (held - (-n // BLOCK)) // 8))
     if splits > 1:
         ws = torch.empty(lib.nsn_prefill_workspace_floats(B, Hq, Hkv, n, splits), dtype=torch.float32, device=q.device)
     rc = lib.nsn_prefill_attention_split(a, splits, ws if ws is None else ws.data_ptr(), _dev.stream())

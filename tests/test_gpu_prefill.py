@@ -181,6 +181,32 @@ def test_prefill_context_splits(monkeypatch, splits, Hq, n, dtype, bits):
     run_case(43, 3, Hq, 2, [300, 1050, 2500], n, bits, dtype)
 
 
+@pytest.mark.parametrize("blocks,tail,n,splits", [(11, 640, 128, 1), (13, 640, 64, 2), (14, 640, 128, 2), (0, 1536, 64, 2)])
+def test_prefill_splits_of_unknown_lengths(monkeypatch, blocks, tail, n, splits):
+    """Lengths that stay on the device: as many splits as the packed capacity,
+    two blocks of tail and the chunk fill; a long tail's empty room does not
+    count, and a context without packed blocks counts all of it."""
+    lib, used = kernels._lib.lib(), []
+    real = lib.nsn_prefill_attention_split
+
+    def launch(a, s, ws, stream):
+        used.append(s)
+        return real(a, s, ws, stream)
+    monkeypatch.setattr(lib, "nsn_prefill_attention_split", launch)
+    rng = np.random.default_rng(47)
+    sides = []
+    for _ in range(2):
+        kv, seq = cache.pack_sequences(torch.from_numpy(normal_tokens(rng, (1, 8), max(64 * blocks, 64))).to(DEV),
+                                       [max(64 * blocks, 64)], tail_dtype=torch.float16)
+        kv.tail = torch.zeros((1, 8, tail, 128), dtype=torch.float16, device=DEV)
+        if not blocks:
+            kv = kernels.PackedKV(None, None, None, None, None, None, kv.tail, 3)
+        sides.append(kv)
+    q, kc, vc = (torch.from_numpy(normal_tokens(rng, (1, h), n)).to(DEV) for h in (32, 8, 8))
+    kernels.prefill_attention(q, sides[0], sides[1], seq, kc, vc, check=False)
+    assert used == [splits]
+
+
 def test_prefill_context_splits_append(monkeypatch):
     """The splits of the last tile append the chunk between them: tails and
     status as without splits, output within one rounding of it."""
