@@ -170,6 +170,32 @@ def test_prefill_tiles_across_heads(Hq, Hkv, n):
     run_case(42, 2, Hq, Hkv, [200, 70], n, 3, torch.float16)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,n", [(1, 6, 2, 85), (2, 32, 8, 300), (2, 64, 2, 256), (2, 65, 5, 256), (3, 28, 4, 600)])
+def test_prefill_tiles_of_single_heads(B, Hq, Hkv, n):
+    """A call whose q-heads' tiles fit the 256 CUs has one head a tile (128 and
+    256 of them; 260 and 252 around the limit), an append by one head of each
+    group; the oracle's output and the tails as without the append's launch."""
+    rng = np.random.default_rng(46)
+    L = [200] * B
+    x = [torch.from_numpy(normal_tokens(rng, (B, Hkv), 200)).to(DEV) for _ in range(2)]
+    q, kc, vc = (torch.from_numpy(normal_tokens(rng, (B, h), n)).to(DEV) for h in (Hq, Hkv, Hkv))
+    sides = []
+    for t in x:
+        kv, seq = cache.pack_sequences(t, L, tail_dtype=torch.float16)
+        room = torch.zeros((B, Hkv, 64 + n, 128), dtype=torch.float16, device=DEV)
+        room[:, :, :kv.tail.shape[2]] = kv.tail
+        kv.tail = room
+        sides.append(kv)
+    out = kernels.prefill_attention(q, sides[0], sides[1], seq, kc, vc, append=True).float().cpu().numpy()
+    for kv, new in zip(sides, (kc, vc)):
+        assert torch.equal(kv.tail[:, :, 8:8 + n], new) and not bool(kv.tail[:, :, 8 + n:].any())
+    for b in range(B):
+        ctx = [restore_ctx(t[b].cpu().numpy(), 200, 3, torch.float16) for t in x]
+        ref = O.prefill_attention64(*(a.float().cpu().numpy() if torch.is_tensor(a) else a
+                                      for a in (q[b], *ctx, kc[b], vc[b])))
+        assert np.all(np.abs(out[b] - ref) <= ATOL + (RTOL + 2.0 ** -11) * np.abs(ref))
+
+
 @pytest.mark.parametrize("dtype,bits", [(torch.bfloat16, 3), (torch.float16, 5)])
 @pytest.mark.parametrize("splits,Hq,n", [(2, 4, 70), (3, 2, 1), (5, 4, 300), (16, 2, 33)])
 def test_prefill_context_splits(monkeypatch, splits, Hq, n, dtype, bits):
@@ -233,25 +259,27 @@ def test_prefill_context_splits_append(monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("where,Hq,n,L,splits", [
-    ("k_factors", 2, 90, 1920, 4),   # every block of the second of four splits: NaN scores only
-    ("k_chunk", 1, 512, 512, 2),     # a NaN key in each chunk block; the later tile's second split is the chunk
-    ("v_chunk", 3, 600, 384, 2),     # a NaN value in a split where the earlier queries of a head see no token
-    ("v_factors", 2, 90, 1920, 4),
+@pytest.mark.parametrize("where,B,Hq,n,L,splits", [
+    ("k_factors", 1, 2, 90, 1920, 4),   # every block of the second of four splits: NaN scores only
+    ("k_chunk", 1, 1, 512, 512, 2),     # a NaN key in each chunk block; the later tile's second split is the chunk
+    # a NaN value in a split where the earlier queries of a head see no token
+    # (32 sequences: the unsplit call's tiles run over head ends as well)
+    ("v_chunk", 32, 3, 600, 384, 2),
+    ("v_factors", 1, 2, 90, 1920, 4),
 ])
-def test_prefill_context_splits_keep_nonfinite_values(monkeypatch, where, Hq, n, L, splits, dtype):
+def test_prefill_context_splits_keep_nonfinite_values(monkeypatch, where, B, Hq, n, L, splits, dtype):
     """Nonfinite K/V in one split only: the NaN outputs and the status are those
     of the unsplit call, the other rows within one rounding of the output and
     one of the weights (whose scale moves with the split's maximum)."""
     from nsn_amd import _dev, _lib
     rng = np.random.default_rng(45)
-    (kk, seq), (vv, _) = (cache.pack_sequences(torch.from_numpy(normal_tokens(rng, (1, 1), L)).to(DEV), [L],
+    (kk, seq), (vv, _) = (cache.pack_sequences(torch.from_numpy(normal_tokens(rng, (B, 1), L)).to(DEV), [L] * B,
                                                tail_dtype=dtype) for _ in range(2))
-    q, kc, vc = (torch.from_numpy(normal_tokens(rng, (1, h), n)).to(DEV, dtype) for h in (Hq, 1, 1))
+    q, kc, vc = (torch.from_numpy(normal_tokens(rng, (B, h), n)).to(DEV, dtype) for h in (Hq, 1, 1))
     if where == "k_factors":
-        kk.factor.view(1, 1, -1, 64)[:, :, 8:16] = float("nan")
+        kk.factor.view(B, 1, -1, 64)[:, :, 8:16] = float("nan")
     elif where == "v_factors":
-        vv.factor.view(1, 1, -1, 64)[:, :, 8:16] = float("nan")
+        vv.factor.view(B, 1, -1, 64)[:, :, 8:16] = float("nan")
     elif where == "k_chunk":
         kc[:, :, ::64] = float("nan")
     else:
