@@ -333,10 +333,9 @@ extern "C" int nsn_kscore(const nsn_kscore_args *a, nsn_stream_t stream) {
     // tokens: u8 129.2 -> 122.4 us, 3-bit 73.2 -> 69.8 us; short calls would
     // lose: 3 x 7.8K tokens in 8-tile runs or finer 9.3 -> 15.7 us).
     int64_t chunk = (streams * tiles + 4095) / 4096;
-    const int64_t least = D / 16;
-    if (chunk >= 4 * least) {
+    if (chunk >= D / 4) {
         chunk = (streams * tiles + 16383) / 16384;
-        chunk = chunk < least ? least : (chunk > 64 ? 64 : chunk);
+        chunk = chunk > 64 ? 64 : chunk;
     }
     const int64_t n_chunks = (tiles + chunk - 1) / chunk;
     const int64_t waves = streams * n_chunks;

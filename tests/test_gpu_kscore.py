@@ -115,12 +115,21 @@ def test_kscore_reference_golden_scores(recipe, bits):
     assert np.abs(got - ref).max() <= REL_MAX * np.abs(ref).max()
 
 
-@pytest.mark.parametrize("fp16", [False, True])
-def test_kscore_short_runs_match_single_sequences(fp16):
+def _run(streams, tiles, D):
+    """16-token tiles of a wave's run (the rule of nsn_kscore's launch)."""
+    n = -(-streams * tiles // 4096)
+    return min(64, -(-streams * tiles // 16384)) if n >= D // 4 else min(64, n)
+
+
+@pytest.mark.parametrize("fp16,B,D", [(False, 6, 128), (True, 6, 128), (False, 8, 256)])
+def test_kscore_short_runs_match_single_sequences(fp16, B, D):
     """A call large enough for four rounds of shorter runs (the last tile of
     each sequence partial), and queries, steps and minima at 2-byte
-    alignments: bit for bit the scores of one sequence at a time."""
-    B, n_kv, D, n_q, T = 4, 16, 128, 32, 32773
+    alignments: bit for bit the scores of one sequence at a time, whose runs
+    are of another length."""
+    n_kv, n_q, T = 16, 32, 32773
+    tiles = -(-T // 16)
+    assert B * n_kv * tiles >= 4096 * (D // 4 - 1) + 1 and _run(B * n_kv, tiles, D) != _run(n_kv, tiles, D)
     g = torch.Generator(device=DEV).manual_seed(5)
 
     def odd(shape, scale):   # contiguous, 2 bytes past a 16-byte boundary
