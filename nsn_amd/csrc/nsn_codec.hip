@@ -617,8 +617,12 @@ struct RestoreParams {
     int32_t *status;
 };
 
-// STREAM: an output past the L2s' 32 MB is stored with the non-temporal hint
-// (266 MB of bf16: 77.0 -> 70.8 us); a smaller one stays in them for its reader.
+// STREAM: an output past the L2s' 32 MB is stored with the non-temporal hint; a
+// smaller one stays in them for its reader.  Alone, then with a dense decode
+// that reads the output at once, then with a copy of it, without -> with the
+// hint: 64 MB 23.9 -> 22.1, 50.3 -> 51.0, 43.5 -> 44.8 us; 128 MB 39.2 -> 38.3,
+// 102.0 -> 94.8, 78.5 -> 83.9; 256 MB 80.4 -> 73.6, 205 -> 176, 181 -> 170; 510
+// MB 153 -> 141, 380 -> 326, 349 -> 333.
 template <int BITS, int OUT_DT, int TAIL_DT, bool STREAM>
 __global__ __launch_bounds__(256) void restore_kernel(RestoreParams p) {
     using TO = typename Elem<OUT_DT>::T;

@@ -38,8 +38,8 @@
 // with everything overlapped and ~5200 one after the other.  The two waves of
 // a SIMD therefore run half a block out of step (see the block loop).  A late
 // 512-query chunk of a batch (32 sequences, 16 heads, 7680 tokens of context)
-// took 1271 us with 16x16x32 tiles and both waves in step, 1185 us so (at 1.8
-// GHz under the full load); one sequence of 32K tokens, 32 query heads, which
+// took 1260 us with 16x16x32 tiles and both waves in step, 1160 us so (in turn
+// on one box, 1146-1213 us over boxes, at 1.8 GHz under the full load); one sequence of 32K tokens, 32 query heads, which
 // loads a quarter of the CUs at 2.3 GHz, 1206 -> 873 us.
 #include <type_traits>
 
@@ -453,8 +453,9 @@ __device__ __forceinline__ void fill_packed(const uint8_t *st, int rg, int cg, c
 // PV product and the row sums as bf16 hi + lo (~2^-17 relative) instead of
 // one bf16 rounding (2^-9) -- for chunks with little or no context, whose
 // first queries attend a handful of tokens, where one weight's bf16 rounding
-// moves the output by up to 2^-9 of |v|.  It costs ~24 % more time per
-// block (36 more MFMA and ~80 more VALU per wave), so the caller asks for it.
+// moves the output by up to 2^-9 of |v|.  It costs 16 more MFMA and the split
+// of 32 weights per wave and block (a late chunk 1160 -> 1640 us, the first
+// chunk 119 -> 138 us), so the caller asks for it.
 template <int BITS, int DT, int TDT, bool LO>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))) void prefill_kernel(PrefillParams p) {
     using S = Stage<BITS>;
@@ -751,7 +752,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     // Priorities: a fill goes before the other wave's softmax (and its own
     // products come right behind it), so that the products overlap the rest of
     // that softmax; without priorities the older waves win every conflict and
-    // the late chunk takes 1224 us instead of 1160.  The packed stretch (blocks
+    // the late chunk takes 6 % longer.  The packed stretch (blocks
     // j .. j + 2 packed) has a loop of its own: its body has no branch on the
     // block kind.
     auto attend = [&](auto packed_c, int j) __attribute__((always_inline)) {

@@ -138,10 +138,10 @@ def decode_split(batch, heads_kv, max_len, kernel, group=1):
     cut finer (_finest_split) where that leaves a wave fewer blocks to walk in
     series, which is what bounds a short context.  The fast kernel takes one
     slot more than there are splits: its blocks per wave are bounded by blocks /
-    (slots - 1).  Kernel times, default_split -> this: fast 1 x 16 kv-heads x
-    1023 tokens 15.7 -> 11.3 us, 5 x 4 x 6500 (7 queries each) 20.0 -> 18.3,
-    64 x 8 x 500 22.3 -> 17.6; exact-order 4 x 8 x 2000 48.1 -> 31.3, 1 x 8 x
-    4133 48.2 -> 21.2.
+    (slots - 1).  Split + merge without host work, default_split -> this: fast
+    1 x 16 kv-heads x 1000 tokens 17.3 -> 11.3 us, 5 x 4 x 6500 (7 queries each)
+    20.0 -> 18.3, 64 x 8 x 490 22.3 -> 16.6; exact-order 4 x 8 x 2000 48.1 ->
+    31.3, 1 x 8 x 4000 48.2 -> 21.2.
     """
     split, n = default_split(batch, heads_kv, max_len)
     blocks = -(-max_len // BLOCK) or 1
@@ -344,8 +344,8 @@ def prefill_attention(q, k: Optional[PackedKV], v: Optional[PackedKV], ctx_len, 
     (loop_kv_pk01_cache.py:101-102) that otherwise follows as a separate
     append; k and v must then carry tails with room for n more tokens.
     ``precise_weights`` (bf16 only): the softmax weights enter the PV product
-    as bf16 hi + lo (~2^-17 relative) instead of one bf16 rounding, at ~24 %
-    more kernel time; None = only when there is no context (k is None), where
+    as bf16 hi + lo (~2^-17 relative) instead of one bf16 rounding, at 16 %
+    (no context) to 41 % (a late chunk) more kernel time; None = only when there is no context (k is None), where
     the first queries attend a handful of tokens.
 
     Where the call has few tiles for its context, the context is split and the
