@@ -276,6 +276,9 @@ int nsn_decode_attention_static(const nsn_attn_args *args, nsn_stream_t stream);
  * tail dtype -- what nsn_tail_append_cast writes.  Needs both tails; a
  * sequence whose tail lacks the room raises NSN_ST_CAPACITY and is not
  * appended.
+ * A nonfinite output raises NSN_ST_NONFINITE_OUTPUT.  A nonfinite V value of a
+ * chunk token reaches every query that attends it, and may reach others of the
+ * call whose weight for it is 0 (0 * NaN).
  * Needs k.blocks and v.blocks equal per sequence (or both NULL), decode
  * factors, 16-byte aligned arrays, one dtype for q, the chunk K/V and out,
  * and one tail dtype (fp16 or bf16) for both tails.
